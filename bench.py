@@ -54,7 +54,7 @@ WORKLOADS = {
     # (the same FLOPs as c3)
     "d256": dict(name="c3 sequence at head_dim 256", B=1, H=20, S=40960, D=256,
                  block=(4, 8, 8), topk=20, gate="full"),
-    # not a BASELINE row: the c3 shape with fp32 inputs (fp32 vector-ALU kernels)
+    # not a BASELINE row: the c3 shape with fp32 inputs (the fp32 kernels)
     "c3f32": dict(name="Video-DiT mid shape in fp32", B=1, H=40, S=40960, D=128,
                   block=(4, 8, 8), topk=20, gate="full", dtype="fp32"),
 }

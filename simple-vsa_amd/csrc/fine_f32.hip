@@ -1,25 +1,34 @@
 // Sparse fine forward, dQ and dK/dV for fp32 inputs (the reference's GPU path
-// accepts fp32: triton_impl.py:375-376).  Every product and sum stays fp32
-// (no operand rounding): outputs, LSE (base 2), the fused combine, the
-// pooled-gradient folds and the padding masks follow the bf16 / fp16 kernels
-// of fine_fwd.hip and fine_bwd.hip with T = fp32.
+// accepts fp32: triton_impl.py:375-376).  Inputs, sums and results are fp32:
+// outputs, LSE (base 2), the fused combine, the pooled-gradient folds and the
+// padding masks follow the bf16 / fp16 kernels of fine_fwd.hip and
+// fine_bwd.hip with T = fp32.
 //
-// The products run on v_mfma_f32_32x32x2_f32 (the fp32 matrix core: 1/16 of
-// the bf16 rate, twice the unpacked fp32 VALU rate).  Its operands are one
-// float per lane:
+// Head dims 64 / 128 run their products on the bf16
+// matrix core: every fp32 operand is the exact sum of three bf16 values, each
+// the upper half of what the ones before leave (mid < 2^-7 hi, lo < 2^-15 hi),
+// and a product is its six largest partial products, accumulated in fp32
+// (mid.lo and lo.mid, on average 2^-25 of the product, are left out: half an
+// fp32 rounding).  A 32x32 tile over 16 dims takes 6 x 32 cycles against
+// 8 x 64 on v_mfma_f32_32x32x2_f32, and its sum is rounded 6 times instead of
+// 16.  Bound by the matrix core: at 12 heads, 16 384 tokens, head dim 128,
+// block 256, topk 8 the forward takes 1.31 ms against 2.89 on the fp32 units,
+// dQ 1.65 against 2.85, dK/dV 2.47 against 4.31 (950 - 1 130 TFLOP/s of bf16
+// products; a large bf16 matrix product reaches 1 126 on this card), and the
+// error against fp64 is 1.0e-6 against 1.1e-6.
+//
+// The forward and dQ at head_dim 256 (split fragments would exceed a wave's
+// registers) run on
+// v_mfma_f32_32x32x2_f32 (the fp32 matrix core: 1/16 of the bf16 rate, twice
+// the unpacked fp32 VALU rate).  Its operands are one float per lane:
 //   A (32 x 2): lane (r, h) = row r, k = h;  B (2 x 32): lane (c, h) = column c, k = h;
 //   C (32 x 32): element i of lane (c, h) = row 8(i/4) + 4h + i%4, column c.
 // A dot product over D dims is D/2 MFMAs; k-step t pairs dim t (h = 0) with
 // dim D/2 + t (h = 1), so each lane reads its row contiguously.  The C tile of
 // one product is the B operand of the next with no data movement (element t of
 // the accumulator is the k = h value of k-step t, rows 8(t/4) + 4h + t%4), and
-// the other operand is read in that row order.
-//
-// Work decomposition as in the bf16 kernels: 32 rows (queries, or keys for
-// dK/dV) per wave, two waves per workgroup; the streamed operand goes through
-// LDS in 32-row chunks (rows padded by 4 floats so that the row reads of 32
-// lanes hit distinct banks).  dK/dV at head_dim 256 (whose fragments and
-// accumulators would exceed a wave's registers) keeps a vector-ALU kernel.
+// the other operand is read in that row order.  dK/dV at head_dim 256 keeps a
+// vector-ALU kernel.
 #include "fine_f32.h"
 #include "vsa_device.h"
 #include "vsa_launch.h"
@@ -54,33 +63,6 @@ __device__ __forceinline__ void stage32(float* dst, const float* __restrict__ sr
     *reinterpret_cast<f32x4*>(dst + r * LD + 4 * c) = val;
   }
 }
-
-// stage32 split in two: load() issues this thread's loads of a 32-row tile
-// into registers, store() writes them to LDS, so the next chunk's loads are in
-// flight while the current one is multiplied (for kernels at one wave per
-// SIMD, where no other wave of the SIMD hides the copy).
-template <int D, int LD, int NT>
-struct Stage32 {
-  static constexpr int V4 = D / 4;
-  static constexpr int N = kChunk * V4 / NT;  // float4 per thread
-  static_assert(kChunk * V4 % NT == 0, "tile must split evenly over the workgroup");
-  f32x4 buf[N];
-  __device__ __forceinline__ void load(const float* __restrict__ src, int valid) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int x = (int)threadIdx.x + i * NT, r = x / V4, c = x % V4;
-      buf[i] = r < valid ? *reinterpret_cast<const f32x4*>(src + (int64_t)r * D + 4 * c)
-                         : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  __device__ __forceinline__ void store(float* dst) const {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int x = (int)threadIdx.x + i * NT, r = x / V4, c = x % V4;
-      *reinterpret_cast<f32x4*>(dst + r * LD + 4 * c) = buf[i];
-    }
-  }
-};
 
 // Copy `rows` rows of D floats (row stride D) into LDS (row stride D) with 256
 // threads; rows past `valid` are zero.
@@ -134,26 +116,687 @@ __device__ __forceinline__ void mma_cols(f32x16 (&acc)[D / 32], const float* lds
 
 }  // namespace
 
+// ---------------------------------------------------------------------------
+// Split-bf16 products
+// ---------------------------------------------------------------------------
+namespace {
+
+typedef __bf16 bf16_t;
+
+// Eight fp32 values as three bf16 MFMA operands.
+struct Split8 {
+  bf16x8 hi, mid, lo;
+};
+
+// The upper halves of two floats, packed.
+__device__ __forceinline__ uint32_t pack_hi16(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ float trunc16(float x) {
+  return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+}
+
+// x = hi + mid + lo of a finite x, each the truncation of what is left: the
+// differences are exact and the last one has 8 significant bits.
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+  u32x4 hi, mid, lo;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float a = x[2 * e], b = x[2 * e + 1];
+    const float a1 = a - trunc16(a), b1 = b - trunc16(b);
+    const float a2 = a1 - trunc16(a1), b2 = b1 - trunc16(b1);
+    hi[e] = pack_hi16(a, b);
+    mid[e] = pack_hi16(a1, b1);
+    lo[e] = pack_hi16(a2, b2);
+  }
+  return {as_vec8<bf16_t>(hi), as_vec8<bf16_t>(mid), as_vec8<bf16_t>(lo)};
+}
+
+// Largest magnitude of the eight (a NaN stays a NaN): split8 needs it finite.
+__device__ __forceinline__ float absmax8(const float (&x)[8]) {
+  float mx = fabsf(x[0]);
+#pragma unroll
+  for (int e = 1; e < 8; ++e) mx = vmax(mx, fabsf(x[e]));
+  return mx;
+}
+
+// split8 of any values: an infinity or NaN goes into the lo part alone.  lo
+// only meets the other operand's hi part, so inf * y is an infinity of the
+// right sign (NaN for y = 0) as in fp32, where an infinite hi would also meet
+// the zeros and signs of the other operand's mid and lo parts.
+__device__ __forceinline__ Split8 split8_any(const float (&x)[8]) {
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = fabsf(x[e]) < INFINITY ? x[e] : 0.f;
+  Split8 s = split8(y);
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (!(fabsf(x[e]) < INFINITY)) s.lo[e] = (bf16_t)x[e];
+  return s;
+}
+
+// acc += a . b over 16 dims: the six partial products, the small ones first.
+__device__ __forceinline__ f32x16 mma6(const Split8& a, const Split8& b, f32x16 acc) {
+  using E = Elem<bf16_t>;
+  acc = E::mfma32(a.lo, b.hi, acc);
+  acc = E::mfma32(a.hi, b.lo, acc);
+  acc = E::mfma32(a.mid, b.mid, acc);
+  acc = E::mfma32(a.mid, b.hi, acc);
+  acc = E::mfma32(a.hi, b.mid, acc);
+  return E::mfma32(a.hi, b.hi, acc);
+}
+
+// This lane's row of an operand held in registers: dims 16 ks + 8h .. +7.
 template <int D>
-struct F32Cfg {
-  static constexpr int LD = D + 4;                 // LDS row stride (floats)
-  static constexpr int NT = 128;                   // two waves
-  // waves per SIMD the registers are sized for: forward and dQ hold two D/2
-  // fragments or accumulators of D/32 tiles, dK/dV four
-  static constexpr int WPE_FWD = D <= 128 ? 2 : 1;
-  static constexpr int WPE_DQ = D <= 64 ? 2 : 1;
-  static constexpr int WPE_KV = D <= 64 ? 2 : 1;
+__device__ __forceinline__ void load_split(Split8 (&f)[D / 16], const float* __restrict__ row,
+                                           int h) {
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      const f32x4 t = *reinterpret_cast<const f32x4*>(row + 16 * ks + 8 * h + e);
+      x[e] = t[0]; x[e + 1] = t[1]; x[e + 2] = t[2]; x[e + 3] = t[3];
+    }
+    f[ks] = split8_any(x);
+  }
+}
+
+// A streamed tile of 32 rows in LDS: three bf16 planes, each swizzled as the
+// bf16 kernels' tiles.
+template <int D>
+struct SplitTile {
+  static constexpr int PLANE = kChunk * D;    // elements
+  static constexpr int ELEMS = 3 * PLANE;
+};
+
+// The copy of a 32-row tile: load() issues this thread's global loads, put(i)
+// splits piece i (8 floats of one row) and writes it to the three planes.  The
+// pieces are put between the MFMAs of the product before the tile's own, with
+// no branch among them; finish() writes the tile again, value by value, in the
+// rare case that it holds an infinity or NaN.
+template <int D, int NT>
+struct SplitCopy {
+  static constexpr int N = kChunk * D / 8 / NT;
+  static_assert(N >= 1 && kChunk * D / 8 % NT == 0, "tile must split evenly over the workgroup");
+  f32x4 buf[N][2];
+  float mx;  // largest magnitude put so far
+  // rows past `valid` are zero (never used for a valid result, only kept finite)
+  __device__ __forceinline__ void load(const float* __restrict__ src, int valid) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int x = (int)threadIdx.x + i * NT, r = x / (D / 8), c = x % (D / 8);
+      const f32x4* p = reinterpret_cast<const f32x4*>(src + r * D + 8 * c);
+      const bool on = r < valid;
+      buf[i][0] = on ? p[0] : f32x4{0.f, 0.f, 0.f, 0.f};
+      buf[i][1] = on ? p[1] : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    mx = 0.f;
+  }
+  __device__ __forceinline__ void store(int i, const Split8& s, bf16_t* tile) const {
+    const int x = (int)threadIdx.x + i * NT;
+    bf16_t* dst = tile + swz<D>(x / (D / 8), x % (D / 8));
+    *reinterpret_cast<bf16x8*>(dst) = s.hi;
+    *reinterpret_cast<bf16x8*>(dst + SplitTile<D>::PLANE) = s.mid;
+    *reinterpret_cast<bf16x8*>(dst + 2 * SplitTile<D>::PLANE) = s.lo;
+  }
+  __device__ __forceinline__ void put(int i, bf16_t* tile) {
+    const float v[8] = {buf[i][0][0], buf[i][0][1], buf[i][0][2], buf[i][0][3],
+                        buf[i][1][0], buf[i][1][1], buf[i][1][2], buf[i][1][3]};
+    mx = vmax(mx, absmax8(v));
+    store(i, split8(v), tile);
+  }
+  __device__ __forceinline__ void finish(bf16_t* tile) const {
+    if (!__any(!(mx < INFINITY))) return;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float v[8] = {buf[i][0][0], buf[i][0][1], buf[i][0][2], buf[i][0][3],
+                          buf[i][1][0], buf[i][1][1], buf[i][1][2], buf[i][1][3]};
+      store(i, split8_any(v), tile);
+    }
+  }
+  __device__ __forceinline__ void put_all(bf16_t* tile) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) put(i, tile);
+    finish(tile);
+  }
+  // piece to put after step `st` of `of` product steps (spread from step
+  // `first` on); -1: none
+  static __device__ __forceinline__ constexpr int piece_after(int st, int of, int first) {
+    const int per = (of - first) / N;
+    return st >= first && (st - first) % per == per - 1 && (st - first) / per < N
+               ? (st - first) / per : -1;
+  }
+};
+
+// Row r of the tile, dims 16 ks + 8h .. +7.
+template <int D>
+__device__ __forceinline__ Split8 tile_row(const bf16_t* tile, int r, int ks, int h) {
+  Split8 s;
+  s.hi = row_a8<bf16_t, D>(tile, r, ks, h);
+  s.mid = row_a8<bf16_t, D>(tile + SplitTile<D>::PLANE, r, ks, h);
+  s.lo = row_a8<bf16_t, D>(tile + 2 * SplitTile<D>::PLANE, r, ks, h);
+  return s;
+}
+
+// Dims d0 .. d0+31 of the tile's rows 16 kk + (the C tile's row order).
+template <int D>
+__device__ __forceinline__ Split8 tile_col(const bf16_t* tile, int d0, int kk) {
+  Split8 s;
+  s.hi = tr_a8<bf16_t, D>(tile, d0, 16 * kk, 16 * kk + 8);
+  s.mid = tr_a8<bf16_t, D>(tile + SplitTile<D>::PLANE, d0, 16 * kk, 16 * kk + 8);
+  s.lo = tr_a8<bf16_t, D>(tile + 2 * SplitTile<D>::PLANE, d0, 16 * kk, 16 * kk + 8);
+  return s;
+}
+
+// Half kk of a C tile (16 of its rows) as the other operand of the next product.
+__device__ __forceinline__ Split8 split_acc(const f32x16& acc, int kk) {
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = acc[8 * kk + e];
+  return split8(x);
+}
+
+// Steps 0 .. N-1 of a product: step st's LDS operand `load(st)` is read one step
+// ahead of its use in `mul(st, operand)`.  The scheduler keeps to the steps (it
+// would otherwise read many operands ahead and spill).
+template <int N, typename L, typename M>
+__device__ __forceinline__ void pipelined(L load, M mul) {
+  Split8 cur = load(0);
+#pragma unroll
+  for (int st = 0; st < N; ++st) {
+    Split8 next = cur;
+    if (st + 1 < N) next = load(st + 1);
+    mul(st, cur);
+    cur = next;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+}  // namespace
+
+// Rows per workgroup: 128 in four waves, or the 64 of a small block in two.
+template <int D, int BE>
+struct SplitCfg {
+  static constexpr int ROWS = BE >= 128 ? 128 : 64;
+  static constexpr int NT = 2 * ROWS;
+  // waves per SIMD the registers are sized for: the fragments of a row take
+  // 3 D/4 registers (one operand in the forward, two backward)
+  // backward: the tiles' loads are issued one product ahead of the product they
+  // are put under; a two-wave workgroup (twice the registers of loads a thread)
+  // issues them as that product starts
+  static constexpr bool EARLY = NT == 256;
+  static constexpr int FIRST = EARLY ? 0 : D / 32;
+  // dK/dV at head_dim 128: the lo parts of the workgroup's V stay in LDS (its
+  // fragments and accumulators would take 24 registers too many), and a
+  // two-wave workgroup, of which two share a CU, keeps one Q buffer
+  static constexpr bool VLO = D == 128;
+  static constexpr int QBUF = VLO && NT == 128 ? 1 : 2;
+  static constexpr int WPE_FWD = D == 64 ? 2 : 1;
+  static constexpr int WPE_DQ = D == 64 && BE >= 128 ? 2 : 1;
+};
+
+// Chunk cursor over a query block's route: slot s, key block kv with nvb valid
+// keys, first key c0.
+template <int BE>
+struct RouteCursor {
+  const int32_t* sel;
+  const int32_t* vbs;
+  int topk, kb;
+  int s = -1, kv = 0, nvb = 0, c0 = 0;
+  __device__ __forceinline__ bool next() {
+    c0 += kChunk;
+    while (c0 >= nvb) {
+      if (++s >= topk) return false;
+      kv = sel[s];
+      nvb = (kv >= 0 && kv < kb) ? clamp_valid(vbs[kv], BE) : 0;
+      c0 = 0;
+    }
+    return true;
+  }
+  __device__ __forceinline__ int row() const { return kv * BE + c0; }
+  __device__ __forceinline__ int keys() const { return min(kChunk, nvb - c0); }
 };
 
 // ---------------------------------------------------------------------------
 // Forward: out = softmax(q k^T scale) v over the selected blocks, LSE base 2,
+// combine `out_c * gate` in the epilogue.  Per wave (32 queries) and 32-key
+// chunk: S^T = K Q^T, online softmax per lane-query (lane halves hold 16 keys
+// each, joined by a permlane swap), O^T += V^T P^T.  The exponents' offset is
+// kSplitSlack above a row's max when it moves, and moves only when a chunk
+// passes it: weights stay <= 1 and O is rescaled on few chunks.  The next V tile is split and written under
+// the S products, the next K tile under the O products: one buffer each and
+// two barriers a chunk.
+// ---------------------------------------------------------------------------
+constexpr float kSplitSlack = 8.0f;
+
+template <int D, int BE>
+__global__ __launch_bounds__((SplitCfg<D, BE>::NT))
+    __attribute__((amdgpu_waves_per_eu(SplitCfg<D, BE>::WPE_FWD))) void
+    sparse_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                          const float* __restrict__ v, const int32_t* __restrict__ selected,
+                          const int32_t* __restrict__ kv_vbs, float* __restrict__ out,
+                          float* __restrict__ fine, float* __restrict__ lse,
+                          const float* __restrict__ outc, const float* __restrict__ gate,
+                          int gate_mode, int gate_heads, int tiles, int tiles_per_head, int sq,
+                          int skv, int qb, int kb, int topk, float c2) {
+  using C = SplitCfg<D, BE>;
+  using Copy = SplitCopy<D, C::NT>;
+  __shared__ __attribute__((aligned(16))) bf16_t ks_[SplitTile<D>::ELEMS];
+  __shared__ __attribute__((aligned(16))) bf16_t vs_[SplitTile<D>::ELEMS];
+  const int tile = xcd_tile(blockIdx.x, tiles);
+  if (tile >= tiles) return;
+  const int64_t b = tile / tiles_per_head;
+  const int q0 = (tile % tiles_per_head) * C::ROWS;
+  const int qblk = q0 / BE;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 31, h = lane >> 5;
+  const int myq = q0 + wave * 32 + r;
+  const int64_t tok = b * sq + myq;
+  Split8 qf[D / 16];
+  load_split<D>(qf, q + tok * D, h);
+  f32x16 o[D / 32];
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt) o[mt] = f32x16{};
+  float m = -INFINITY, l = 0.f;  // offset of the exponents (log2 units), this half's partial sum
+  const float* kbase = k + b * (int64_t)skv * D;
+  const float* vbase = v + b * (int64_t)skv * D;
+  RouteCursor<BE> cur{selected + (b * qb + qblk) * topk, kv_vbs, topk, kb};
+  Copy cp;
+  bool have = cur.next();
+  if (have) {
+    cp.load(kbase + (int64_t)cur.row() * D, cur.keys());
+    cp.put_all(ks_);
+  }
+  while (have) {
+    const int nk = cur.keys();
+    cp.load(vbase + (int64_t)cur.row() * D, nk);
+    __syncthreads();  // K written; every wave is done with V
+    f32x16 sacc = f32x16{};
+    pipelined<D / 16>([&](int ks) { return tile_row<D>(ks_, r, ks, h); },
+                      [&](int ks, const Split8& a) {
+                        sacc = mma6(a, qf[ks], sacc);
+                        const int i = Copy::piece_after(ks, D / 16, D / 32);
+                        if (i >= 0) cp.put(i, vs_);
+                      });
+    cp.finish(vs_);
+    float cmax = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int key = 8 * (i >> 2) + 4 * h + (i & 3);
+      sacc[i] = key < nk ? sacc[i] * c2 : -INFINITY;
+      cmax = vmax(cmax, sacc[i]);
+    }
+    cmax = pair_max32(cmax);
+    // a row moves its own offset only, so that its values never depend on the
+    // other rows of the wave (a NaN moves it too, and stays)
+    const bool grow = !(cmax <= m);
+    if (__any(grow)) {
+      const float mnew = grow ? cmax + kSplitSlack : m;
+      const float alpha = exp2f(m - mnew);
+      l *= alpha;
+#pragma unroll
+      for (int mt = 0; mt < D / 32; ++mt) o[mt] *= alpha;
+      m = mnew;
+    }
+    float psum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      sacc[i] = exp2f(sacc[i] - m);
+      psum += sacc[i];
+    }
+    l += psum;
+    const Split8 p[2] = {split_acc(sacc, 0), split_acc(sacc, 1)};
+    have = cur.next();
+    if (have) cp.load(kbase + (int64_t)cur.row() * D, cur.keys());
+    __syncthreads();  // V written; every wave is done with K
+    // step x: keys 16 (x / (D/32)) .., dims 32 (x % (D/32)) ..
+    pipelined<D / 16>(
+        [&](int x) { return tile_col<D>(vs_, 32 * (x % (D / 32)), x / (D / 32)); },
+        [&](int x, const Split8& a) {
+          o[x % (D / 32)] = mma6(a, p[x / (D / 32)], o[x % (D / 32)]);
+          const int i = Copy::piece_after(x, D / 16, D / 32);
+          if (i >= 0) cp.put(i, ks_);
+        });
+    cp.finish(ks_);
+  }
+  // epilogue: normalise, fused combine, LSE
+  const float ltot = pair_sum32(l);
+  const float inv = 1.0f / ltot;
+  if (lse != nullptr && h == 0) lse[tok] = m + log2f(ltot);
+  const float* ocrow = outc ? outc + (b * qb + qblk) * D : nullptr;
+  const float* grow = nullptr;
+  float gtok = 1.f;
+  if (outc && gate_mode == 1) grow = gate + tok * D;
+  if (outc && gate_mode == 2) gtok = gate[tok];
+  if (outc && gate_mode == 3)
+    grow = gate + (((b / gate_heads) * sq + myq) * gate_heads + b % gate_heads) * D;
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d0 = 32 * mt + 8 * g + 4 * h;
+      f32x4 val;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) val[e] = o[mt][4 * g + e] * inv;
+      if (ocrow && fine) *reinterpret_cast<f32x4*>(fine + tok * D + d0) = val;
+      if (ocrow) {
+        const f32x4 oc = *reinterpret_cast<const f32x4*>(ocrow + d0);
+        const f32x4 gv = grow ? *reinterpret_cast<const f32x4*>(grow + d0)
+                              : f32x4{gtok, gtok, gtok, gtok};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) val[e] = fmaf(oc[e], gv[e], val[e]);
+      }
+      *reinterpret_cast<f32x4*>(out + tok * D + d0) = val;
+    }
+  }
+}
+
+// dQ rows of a wave from its accumulators: scaled, plus the pooled gradient on
+// the block's valid rows.
+template <int D, int BE>
+__device__ __forceinline__ void store_dq(const f32x16 (&acc)[D / 32], float* __restrict__ dq,
+                                         const float* __restrict__ dqc,
+                                         const int32_t* __restrict__ q_vbs, int64_t b, int64_t tok,
+                                         int myq, int qblk, int qb, int h, float scale) {
+  float cdiv = 1.f;
+  bool cvalid = false;
+  if (dqc) {
+    const int32_t cnt = q_vbs[qblk];
+    cvalid = myq - qblk * BE < clamp_valid(cnt, BE);
+    cdiv = (float)(cnt > 1 ? cnt : 1);
+  }
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d0 = 32 * mt + 8 * g + 4 * h;
+      f32x4 cv = {0.f, 0.f, 0.f, 0.f};
+      if (cvalid) cv = *reinterpret_cast<const f32x4*>(dqc + (b * qb + qblk) * D + d0);
+      f32x4 val;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) val[e] = acc[mt][4 * g + e] * scale + cv[e] / cdiv;
+      *reinterpret_cast<f32x4*>(dq + tok * D + d0) = val;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// dQ (query-owned): per wave (32 queries) and 32-key chunk S^T = K Q^T,
+// dP^T = V dO^T, P^T = exp2(S^T c2 - lse), dS^T = P^T (dP^T - delta),
+// dQ^T += K^T dS^T; dQ = scale dQ plus the pooled gradient d_q_c / count on the
+// block's valid rows.  V is split and written under the S products, the next
+// K tile (a second buffer) under the dP products.
+// ---------------------------------------------------------------------------
+template <int D, int BE>
+__global__ __launch_bounds__((SplitCfg<D, BE>::NT))
+    __attribute__((amdgpu_waves_per_eu(SplitCfg<D, BE>::WPE_DQ))) void
+    sparse_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                         const float* __restrict__ v, const float* __restrict__ dout,
+                         const float* __restrict__ lse, const float* __restrict__ delta,
+                         const int32_t* __restrict__ selected, const int32_t* __restrict__ kv_vbs,
+                         float* __restrict__ dq, const float* __restrict__ dqc,
+                         const int32_t* __restrict__ q_vbs, int tiles, int tiles_per_head, int sq,
+                         int skv, int qb, int kb, int topk, float c2, float scale) {
+  using C = SplitCfg<D, BE>;
+  using Copy = SplitCopy<D, C::NT>;
+  __shared__ __attribute__((aligned(16))) bf16_t ks_[2 * SplitTile<D>::ELEMS];
+  __shared__ __attribute__((aligned(16))) bf16_t vs_[SplitTile<D>::ELEMS];
+  const int tile = xcd_tile(blockIdx.x, tiles);
+  if (tile >= tiles) return;
+  const int64_t b = tile / tiles_per_head;
+  const int q0 = (tile % tiles_per_head) * C::ROWS;
+  const int qblk = q0 / BE;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 31, h = lane >> 5;
+  const int myq = q0 + wave * 32 + r;
+  const int64_t tok = b * sq + myq;
+  Split8 qf[D / 16], df[D / 16];
+  load_split<D>(qf, q + tok * D, h);
+  load_split<D>(df, dout + tok * D, h);
+  const float my_lse = lse[tok], my_delta = delta[tok];
+  f32x16 acc[D / 32];
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt) acc[mt] = f32x16{};
+  const float* kbase = k + b * (int64_t)skv * D;
+  const float* vbase = v + b * (int64_t)skv * D;
+  RouteCursor<BE> cur{selected + (b * qb + qblk) * topk, kv_vbs, topk, kb};
+  Copy kc, vc;
+  int krow = 0;  // first key row of the chunk
+  bool have = cur.next();
+  if (have) {
+    krow = cur.row();
+    kc.load(kbase + (int64_t)krow * D, cur.keys());
+    if (C::EARLY) vc.load(vbase + (int64_t)krow * D, cur.keys());
+    kc.put_all(ks_);
+  }
+  int buf = 0;
+  while (have) {
+    const int nk = cur.keys();
+    const bool more = cur.next();
+    const int row = krow;
+    krow = cur.row();
+    if (C::EARLY && more) kc.load(kbase + (int64_t)krow * D, cur.keys());
+    if (!C::EARLY) vc.load(vbase + (int64_t)row * D, nk);
+    const bf16_t* kt = ks_ + buf * SplitTile<D>::ELEMS;
+    bf16_t* knext = ks_ + (buf ^ 1) * SplitTile<D>::ELEMS;
+    __syncthreads();  // K written; every wave is done with V
+    f32x16 sacc = f32x16{}, pacc = f32x16{};
+    pipelined<D / 16>([&](int ks) { return tile_row<D>(kt, r, ks, h); },
+                      [&](int ks, const Split8& a) {
+                        sacc = mma6(a, qf[ks], sacc);
+                        const int i = Copy::piece_after(ks, D / 16, C::FIRST);
+                        if (i >= 0) vc.put(i, vs_);
+                      });
+    vc.finish(vs_);
+    if (C::EARLY && more) vc.load(vbase + (int64_t)krow * D, cur.keys());
+    if (!C::EARLY && more) kc.load(kbase + (int64_t)krow * D, cur.keys());
+    __syncthreads();  // V written; every wave is done with the other K buffer
+    pipelined<D / 16>([&](int ks) { return tile_row<D>(vs_, r, ks, h); },
+                      [&](int ks, const Split8& a) {
+                        pacc = mma6(a, df[ks], pacc);
+                        const int i = Copy::piece_after(ks, D / 16, C::FIRST);
+                        if (i >= 0) kc.put(i, knext);
+                      });
+    kc.finish(knext);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int key = 8 * (i >> 2) + 4 * h + (i & 3);
+      const float p = key < nk ? exp2f(fmaf(sacc[i], c2, -my_lse)) : 0.f;
+      sacc[i] = p * (pacc[i] - my_delta);
+    }
+    const Split8 ds[2] = {split_acc(sacc, 0), split_acc(sacc, 1)};
+    pipelined<D / 16>(
+        [&](int x) { return tile_col<D>(kt, 32 * (x % (D / 32)), x / (D / 32)); },
+        [&](int x, const Split8& a) {
+          acc[x % (D / 32)] = mma6(a, ds[x / (D / 32)], acc[x % (D / 32)]);
+        });
+    have = more;
+    buf ^= 1;
+  }
+  store_dq<D, BE>(acc, dq, dqc, q_vbs, b, tok, myq, qblk, qb, h, scale);
+}
+
+// ---------------------------------------------------------------------------
+// dK / dV (key-owned over the CSR in-edges of the key block): per wave (32
+// keys) and 32-query item S = Q K^T, dP = dO V^T, P = exp2(S c2 - lse),
+// dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS; dK *= scale; pooled
+// gradients folded on valid keys; padding keys get zero.  dO is split and
+// written under the S products, the next item's Q and statistics (a second
+// buffer) under the dP products.
+// ---------------------------------------------------------------------------
+template <int D, int BE>
+__global__ __launch_bounds__((SplitCfg<D, BE>::NT))
+    __attribute__((amdgpu_waves_per_eu(1))) void
+    sparse_dkdv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                           const float* __restrict__ v, const float* __restrict__ dout,
+                           const float* __restrict__ lse, const float* __restrict__ delta,
+                           const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
+                           const int32_t* __restrict__ inverse, const int32_t* __restrict__ kv_vbs,
+                           float* __restrict__ dk, float* __restrict__ dv,
+                           const float* __restrict__ dkc, const float* __restrict__ dvc, int tiles,
+                           int tiles_per_head, int sq, int skv, int qb, int kb, int topk, float c2,
+                           float scale) {
+  using C = SplitCfg<D, BE>;
+  using Copy = SplitCopy<D, C::NT>;
+  __shared__ __attribute__((aligned(16))) bf16_t qs_[C::QBUF * SplitTile<D>::ELEMS];
+  __shared__ __attribute__((aligned(16))) bf16_t vlo_[C::VLO ? C::ROWS * D : 8];
+  __shared__ __attribute__((aligned(16))) bf16_t os_[SplitTile<D>::ELEMS];
+  __shared__ __attribute__((aligned(16))) float st_[2][2 * kChunk];  // lse, delta of an item
+  const int tile = xcd_tile(blockIdx.x, tiles);
+  if (tile >= tiles) return;
+  const int64_t b = tile / tiles_per_head;
+  const int k0 = (tile % tiles_per_head) * C::ROWS;
+  const int kvblk = k0 / BE;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 31, h = lane >> 5;
+  const int mykey = k0 + wave * 32 + r;
+  const int64_t ktok = b * skv + mykey;
+  const bool key_valid = mykey - kvblk * BE < clamp_valid(kv_vbs[kvblk], BE);
+  Split8 kf[D / 16], vf[D / 16];
+  load_split<D>(kf, k + ktok * D, h);
+  load_split<D>(vf, v + ktok * D, h);
+  if constexpr (C::VLO) {  // each lane reads back what it wrote
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks)
+      *reinterpret_cast<bf16x8*>(vlo_ + swz<D>(wave * 32 + r, 2 * ks + h)) = vf[ks].lo;
+  }
+  f32x16 dka[D / 32], dva[D / 32];
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt) dka[mt] = dva[mt] = f32x16{};
+  const int64_t meta = b * kb + kvblk;
+  const int nedge = counts[meta];
+  const int32_t* seg = inverse + b * (int64_t)qb * topk + offsets[meta];
+  const float* qbase = q + b * (int64_t)sq * D;
+  const float* dbase = dout + b * (int64_t)sq * D;
+  // item it: 32 queries (rows (it % SUBS) * 32 ..) of in-edge query block it / SUBS
+  constexpr int SUBS = BE / kChunk;
+  const int items = nedge * SUBS;
+  auto row_of = [&](int it) { return seg[it / SUBS] * BE + (it % SUBS) * kChunk; };
+  Copy qc, oc;
+  float stv = 0.f;  // lse (threads < 32) or delta (32 .. 63) of the item in qc
+  auto load_q = [&](int row) {
+    qc.load(qbase + (int64_t)row * D, kChunk);
+    if (threadIdx.x < 2 * kChunk)
+      stv = threadIdx.x < kChunk ? lse[b * sq + row + threadIdx.x]
+                                 : delta[b * sq + row + threadIdx.x - kChunk];
+  };
+  int row = 0;  // first query row of the item
+  if (items > 0) {
+    row = row_of(0);
+    load_q(row);
+    if (C::EARLY) oc.load(dbase + (int64_t)row * D, kChunk);
+    qc.put_all(qs_);
+    if (threadIdx.x < 2 * kChunk) st_[0][threadIdx.x] = stv;
+  }
+  for (int it = 0; it < items; ++it) {
+    const int buf = it & 1;
+    const bool more = it + 1 < items;
+    const int next = more ? row_of(it + 1) : 0;
+    if (C::EARLY && more) load_q(next);
+    if (!C::EARLY) oc.load(dbase + (int64_t)row * D, kChunk);
+    const bf16_t* qt = qs_ + (C::QBUF == 2 ? buf : 0) * SplitTile<D>::ELEMS;
+    bf16_t* qnext = qs_ + (C::QBUF == 2 ? buf ^ 1 : 0) * SplitTile<D>::ELEMS;
+    __syncthreads();  // Q and statistics written; every wave is done with dO
+    f32x16 sacc = f32x16{}, pacc = f32x16{};
+    // S (queries x keys), lane column = key r
+    pipelined<D / 16>([&](int ks) { return tile_row<D>(qt, r, ks, h); },
+                      [&](int ks, const Split8& a) {
+                        sacc = mma6(a, kf[ks], sacc);
+                        const int i = Copy::piece_after(ks, D / 16, C::FIRST);
+                        if (i >= 0) oc.put(i, os_);
+                      });
+    oc.finish(os_);
+    if (more && C::EARLY) oc.load(dbase + (int64_t)next * D, kChunk);
+    if (more && !C::EARLY && C::QBUF == 2) load_q(next);
+    row = next;
+    __syncthreads();  // dO written; every wave is done with the other Q buffer
+    pipelined<D / 16>([&](int ks) { return tile_row<D>(os_, r, ks, h); },
+                      [&](int ks, const Split8& a) {
+                        Split8 f = vf[ks];
+                        if constexpr (C::VLO)
+                          f.lo = row_a8<bf16_t, D>(vlo_, wave * 32 + r, ks, h);
+                        pacc = mma6(a, f, pacc);
+                        const int i = Copy::piece_after(ks, D / 16, C::FIRST);
+                        if (C::QBUF == 2 && i >= 0) qc.put(i, qnext);
+                      });
+    if (C::QBUF == 2) qc.finish(qnext);
+    if (C::QBUF == 2 && more && threadIdx.x < 2 * kChunk) st_[buf ^ 1][threadIdx.x] = stv;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 l4 = *reinterpret_cast<const f32x4*>(st_[buf] + 8 * g + 4 * h);
+      const f32x4 d4 = *reinterpret_cast<const f32x4*>(st_[buf] + kChunk + 8 * g + 4 * h);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 4 * g + j;
+        sacc[i] = exp2f(fmaf(sacc[i], c2, -l4[j]));
+        pacc[i] = sacc[i] * (pacc[i] - d4[j]);
+      }
+    }
+    const Split8 p[2] = {split_acc(sacc, 0), split_acc(sacc, 1)};
+    pipelined<D / 16>(  // dV^T += dO^T P
+        [&](int x) { return tile_col<D>(os_, 32 * (x % (D / 32)), x / (D / 32)); },
+        [&](int x, const Split8& a) {
+          dva[x % (D / 32)] = mma6(a, p[x / (D / 32)], dva[x % (D / 32)]);
+        });
+    const Split8 ds[2] = {split_acc(pacc, 0), split_acc(pacc, 1)};
+    pipelined<D / 16>(  // dK^T += Q^T dS
+        [&](int x) { return tile_col<D>(qt, 32 * (x % (D / 32)), x / (D / 32)); },
+        [&](int x, const Split8& a) {
+          dka[x % (D / 32)] = mma6(a, ds[x / (D / 32)], dka[x % (D / 32)]);
+        });
+    if (C::QBUF == 1 && more) {
+      load_q(next);
+      __syncthreads();  // every wave is done with Q and the statistics
+      qc.put_all(qs_);
+      if (threadIdx.x < 2 * kChunk) st_[buf ^ 1][threadIdx.x] = stv;
+    }
+  }
+  const int32_t cnt = kv_vbs[kvblk];
+  const float cdiv = (float)(cnt > 1 ? cnt : 1);
+  // pooled-gradient rows loaded before the first store (a load issued after a
+  // store also waits for that store)
+  f32x4 ckr[D / 32][4], cvr[D / 32][4];
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      ckr[mt][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+      cvr[mt][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (key_valid && dkc) {
+        const int d0 = 32 * mt + 8 * g + 4 * h;
+        ckr[mt][g] = *reinterpret_cast<const f32x4*>(dkc + meta * D + d0);
+        cvr[mt][g] = *reinterpret_cast<const f32x4*>(dvc + meta * D + d0);
+      }
+    }
+#pragma unroll
+  for (int mt = 0; mt < D / 32; ++mt) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d0 = 32 * mt + 8 * g + 4 * h;
+      const f32x4 ck = ckr[mt][g], cv = cvr[mt][g];
+      f32x4 kk, vv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kk[e] = (key_valid ? dka[mt][4 * g + e] * scale : 0.f) + ck[e] / cdiv;
+        vv[e] = (key_valid ? dva[mt][4 * g + e] : 0.f) + cv[e] / cdiv;
+      }
+      *reinterpret_cast<f32x4*>(dk + ktok * D + d0) = kk;
+      *reinterpret_cast<f32x4*>(dv + ktok * D + d0) = vv;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Forward at head_dim 256 on the fp32 matrix core: out = softmax(q k^T scale) v
+// over the selected blocks, LSE base 2,
 // combine `out_c * gate` in the epilogue.  Per wave and 32-key chunk:
 //   S^T = K Q^T (D/2 MFMAs), online softmax per lane-query (lane halves hold
 //   16 keys each, joined by a permlane swap), O^T += V^T P^T (16 D/32 MFMAs).
 // grid: bh * Sq / 64.
 // ---------------------------------------------------------------------------
 template <int D, int BE>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(F32Cfg<D>::WPE_FWD))) void
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1))) void
 sparse_fwd_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
                        const float* __restrict__ v, const int32_t* __restrict__ selected,
                        const int32_t* __restrict__ kv_vbs, float* __restrict__ out,
@@ -161,8 +804,7 @@ sparse_fwd_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
                        const float* __restrict__ outc, const float* __restrict__ gate,
                        int gate_mode, int gate_heads, int tiles_per_head, int sq, int skv, int qb,
                        int kb, int topk, float c2) {
-  using C = F32Cfg<D>;
-  constexpr int LD = C::LD;
+  constexpr int NT = 128, LD = D + 4;  // threads, LDS row stride (floats)
   __shared__ __attribute__((aligned(16))) float ks[kChunk * LD];
   __shared__ __attribute__((aligned(16))) float vs[kChunk * LD];
   const int64_t b = blockIdx.x / tiles_per_head;
@@ -188,8 +830,8 @@ sparse_fwd_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
     for (int c0 = 0; c0 < nvb; c0 += kChunk) {
       const int nk = min(kChunk, nvb - c0);
       __syncthreads();
-      stage32<D, LD, C::NT>(ks, kbase + ((int64_t)kv * BE + c0) * D, nk);
-      stage32<D, LD, C::NT>(vs, vbase + ((int64_t)kv * BE + c0) * D, nk);
+      stage32<D, LD, NT>(ks, kbase + ((int64_t)kv * BE + c0) * D, nk);
+      stage32<D, LD, NT>(vs, vbase + ((int64_t)kv * BE + c0) * D, nk);
       __syncthreads();
       f32x16 sacc = f32x16{};
       mma_rows<D, LD>(sacc, ks, qf, r, h);
@@ -248,13 +890,13 @@ sparse_fwd_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
 }
 
 // ---------------------------------------------------------------------------
-// dQ (query-owned): per wave and 32-key chunk S^T = K Q^T, dP^T = V dO^T,
+// dQ at head_dim 256 (query-owned): per wave and 32-key chunk S^T = K Q^T, dP^T = V dO^T,
 // P^T = exp2(S^T c2 - lse), dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T;
 // dQ = scale dQ plus the pooled gradient d_q_c / count on the block's valid
 // rows.  grid: bh * Sq / 64.
 // ---------------------------------------------------------------------------
 template <int D, int BE>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(F32Cfg<D>::WPE_DQ))) void
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1))) void
 sparse_dq_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
                       const float* __restrict__ v, const float* __restrict__ dout,
                       const float* __restrict__ lse, const float* __restrict__ delta,
@@ -262,8 +904,7 @@ sparse_dq_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
                       float* __restrict__ dq, const float* __restrict__ dqc,
                       const int32_t* __restrict__ q_vbs, int tiles_per_head, int sq, int skv,
                       int qb, int kb, int topk, float c2, float scale) {
-  using C = F32Cfg<D>;
-  constexpr int LD = C::LD;
+  constexpr int NT = 128, LD = D + 4;  // threads, LDS row stride (floats)
   __shared__ __attribute__((aligned(16))) float ks[kChunk * LD];
   __shared__ __attribute__((aligned(16))) float vs[kChunk * LD];
   const int64_t b = blockIdx.x / tiles_per_head;
@@ -294,31 +935,14 @@ sparse_dq_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
     }
     return true;
   };
-  // head_dim <= 128: the next chunk's loads stay in flight under this chunk's
-  // products (64 more registers); head_dim 256 has no registers to spare
-  constexpr bool kPrefetch = D <= 128;
-  Stage32<D, LD, C::NT> kst, vst;
-  auto load_chunk = [&](int kv_, int nvb_, int c0_) {
-    if constexpr (kPrefetch) {
-      kst.load(kbase + ((int64_t)kv_ * BE + c0_) * D, min(kChunk, nvb_ - c0_));
-      vst.load(vbase + ((int64_t)kv_ * BE + c0_) * D, min(kChunk, nvb_ - c0_));
-    }
-  };
   int s = -1, kv = 0, nvb = 0, c0 = 0;
   bool have = advance(s, kv, nvb, c0);
-  if (have) load_chunk(kv, nvb, c0);
   while (have) {
     const int nk = min(kChunk, nvb - c0);
     __syncthreads();
-    if constexpr (kPrefetch) {
-      kst.store(ks);
-      vst.store(vs);
-    } else {
-      stage32<D, LD, C::NT>(ks, kbase + ((int64_t)kv * BE + c0) * D, nk);
-      stage32<D, LD, C::NT>(vs, vbase + ((int64_t)kv * BE + c0) * D, nk);
-    }
+    stage32<D, LD, NT>(ks, kbase + ((int64_t)kv * BE + c0) * D, nk);
+    stage32<D, LD, NT>(vs, vbase + ((int64_t)kv * BE + c0) * D, nk);
     const bool have2 = advance(s, kv, nvb, c0);
-    if (have2) load_chunk(kv, nvb, c0);
     __syncthreads();
     f32x16 sacc = f32x16{}, pacc = f32x16{};
     mma_rows<D, LD>(sacc, ks, qf, r, h);
@@ -332,150 +956,7 @@ sparse_dq_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
     mma_cols<D, LD>(acc, ks, sacc, r, h);
     have = have2;
   }
-  float cdiv = 1.f;
-  bool cvalid = false;
-  if (dqc) {
-    const int32_t cnt = q_vbs[qblk];
-    cvalid = myq - qblk * BE < clamp_valid(cnt, BE);
-    cdiv = (float)(cnt > 1 ? cnt : 1);
-  }
-#pragma unroll
-  for (int mt = 0; mt < D / 32; ++mt) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d0 = 32 * mt + 8 * g + 4 * h;
-      f32x4 cv = {0.f, 0.f, 0.f, 0.f};
-      if (cvalid) cv = *reinterpret_cast<const f32x4*>(dqc + (b * qb + qblk) * D + d0);
-      f32x4 val;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) val[e] = acc[mt][4 * g + e] * scale + cv[e] / cdiv;
-      *reinterpret_cast<f32x4*>(dq + tok * D + d0) = val;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// dK / dV (key-owned over the CSR in-edges of the key block), head_dim 64 /
-// 128: per wave (32 keys) and 32-query item S = Q K^T, dP = dO V^T,
-// P = exp2(S c2 - lse), dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS;
-// dK *= scale; pooled gradients folded on valid keys; padding keys get zero.
-// grid: bh * Skv / 64.
-// ---------------------------------------------------------------------------
-template <int D, int BE>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(F32Cfg<D>::WPE_KV))) void
-sparse_dkdv_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                        const float* __restrict__ v, const float* __restrict__ dout,
-                        const float* __restrict__ lse, const float* __restrict__ delta,
-                        const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
-                        const int32_t* __restrict__ inverse, const int32_t* __restrict__ kv_vbs,
-                        float* __restrict__ dk, float* __restrict__ dv,
-                        const float* __restrict__ dkc, const float* __restrict__ dvc,
-                        int tiles_per_head, int sq, int skv, int qb, int kb, int topk, float c2,
-                        float scale) {
-  using C = F32Cfg<D>;
-  constexpr int LD = C::LD;
-  __shared__ __attribute__((aligned(16))) float qs[kChunk * LD];
-  __shared__ __attribute__((aligned(16))) float os[kChunk * LD];
-  __shared__ __attribute__((aligned(16))) float ls[kChunk], es[kChunk];
-  const int64_t b = blockIdx.x / tiles_per_head;
-  const int k0 = (blockIdx.x % tiles_per_head) * kRows;
-  const int kvblk = k0 / BE;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 31, h = lane >> 5;
-  const int mykey = k0 + wave * 32 + r;
-  const int64_t ktok = b * skv + mykey;
-  const bool key_valid = mykey - kvblk * BE < clamp_valid(kv_vbs[kvblk], BE);
-  float kf[D / 2], vf[D / 2];
-  load_frag<D>(kf, k + ktok * D, h);
-  load_frag<D>(vf, v + ktok * D, h);
-  f32x16 dka[D / 32], dva[D / 32];
-#pragma unroll
-  for (int mt = 0; mt < D / 32; ++mt) dka[mt] = dva[mt] = f32x16{};
-  const int64_t meta = b * kb + kvblk;
-  const int nedge = counts[meta];
-  const int32_t* seg = inverse + b * (int64_t)qb * topk + offsets[meta];
-  const float* qbase = q + b * (int64_t)sq * D;
-  const float* dbase = dout + b * (int64_t)sq * D;
-  // item it: 32 queries (rows (it % (BE/32)) * 32 ..) of in-edge query block it / (BE/32);
-  // head_dim 128: the next item's Q / dO / statistics loads stay in flight
-  // under this item's products (64 more registers; 64 has no headroom at two
-  // waves per SIMD)
-  constexpr int SUBS = BE / kChunk;
-  constexpr bool kPrefetch = D == 128;
-  const int items = nedge * SUBS;
-  Stage32<D, LD, C::NT> qst, ost;
-  float stv = 0.f;  // lse (threads < 32) or delta (32 .. 63) of the staged item
-  auto load_item = [&](int it) {
-    const int qrow0 = seg[it / SUBS] * BE + (it % SUBS) * kChunk;
-    qst.load(qbase + (int64_t)qrow0 * D, kChunk);
-    ost.load(dbase + (int64_t)qrow0 * D, kChunk);
-    if (threadIdx.x < 2 * kChunk)
-      stv = threadIdx.x < kChunk ? lse[b * sq + qrow0 + threadIdx.x]
-                                 : delta[b * sq + qrow0 + threadIdx.x - kChunk];
-  };
-  if (kPrefetch && items > 0) load_item(0);
-  for (int it = 0; it < items; ++it) {
-    {
-      __syncthreads();
-      if (!kPrefetch) load_item(it);
-      qst.store(qs);
-      ost.store(os);
-      if (threadIdx.x < kChunk) ls[threadIdx.x] = stv;
-      else if (threadIdx.x < 2 * kChunk) es[threadIdx.x - kChunk] = stv;
-      if (kPrefetch && it + 1 < items) load_item(it + 1);
-      __syncthreads();
-      f32x16 sacc = f32x16{}, pacc = f32x16{};
-      mma_rows<D, LD>(sacc, qs, kf, r, h);   // S  (queries x keys), lane column = key r
-      mma_rows<D, LD>(pacc, os, vf, r, h);   // dP
-      f32x16 ds;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(ls + 8 * g + 4 * h);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(es + 8 * g + 4 * h);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = 4 * g + j;
-          sacc[i] = exp2f(fmaf(sacc[i], c2, -l4[j]));
-          ds[i] = sacc[i] * (pacc[i] - d4[j]);
-        }
-      }
-      mma_cols<D, LD>(dva, os, sacc, r, h);  // dV^T += dO^T P
-      mma_cols<D, LD>(dka, qs, ds, r, h);    // dK^T += Q^T dS
-    }
-  }
-  const int32_t cnt = kv_vbs[kvblk];
-  const float cdiv = (float)(cnt > 1 ? cnt : 1);
-  // pooled-gradient rows loaded before the first store (a load issued after a
-  // store also waits for that store)
-  f32x4 ckr[D / 32][4], cvr[D / 32][4];
-#pragma unroll
-  for (int mt = 0; mt < D / 32; ++mt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      ckr[mt][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-      cvr[mt][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (key_valid && dkc) {
-        const int d0 = 32 * mt + 8 * g + 4 * h;
-        ckr[mt][g] = *reinterpret_cast<const f32x4*>(dkc + meta * D + d0);
-        cvr[mt][g] = *reinterpret_cast<const f32x4*>(dvc + meta * D + d0);
-      }
-    }
-#pragma unroll
-  for (int mt = 0; mt < D / 32; ++mt) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d0 = 32 * mt + 8 * g + 4 * h;
-      const f32x4 ck = ckr[mt][g], cv = cvr[mt][g];
-      f32x4 kk, vv;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        kk[e] = (key_valid ? dka[mt][4 * g + e] * scale : 0.f) + ck[e] / cdiv;
-        vv[e] = (key_valid ? dva[mt][4 * g + e] : 0.f) + cv[e] / cdiv;
-      }
-      *reinterpret_cast<f32x4*>(dk + ktok * D + d0) = kk;
-      *reinterpret_cast<f32x4*>(dv + ktok * D + d0) = vv;
-    }
-  }
+  store_dq<D, BE>(acc, dq, dqc, q_vbs, b, tok, myq, qblk, qb, h, scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -485,7 +966,7 @@ sparse_dkdv_f32m_kernel(const float* __restrict__ q, const float* __restrict__ k
 // gradients folded on valid keys; padding keys get zero.  grid: bh * Skv / 64.
 // ---------------------------------------------------------------------------
 template <int D, int BE>
-__global__ __launch_bounds__(256) void sparse_dkdv_f32_kernel(
+__global__ __launch_bounds__(256) void sparse_dkdv_f32v_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ dout, const float* __restrict__ lse,
     const float* __restrict__ delta, const int32_t* __restrict__ counts,
@@ -576,18 +1057,27 @@ int sparse_fwd_f32(const void* q, const void* k, const void* v, const int32_t* s
                    const void* gate, int gate_mode, int gate_heads, int64_t bh, int64_t sq,
                    int64_t skv, int D, int be, int topk, float scale, hipStream_t s) {
   if (!f32_shape(D, be)) return VSA_ERR_UNSUPPORTED;
-  const int64_t tiles = bh * (sq / kRows);
-  if (tiles > (1LL << 30)) return VSA_ERR_SHAPE;
-  const int tph = (int)(sq / kRows);
+  if (bh * (sq / kRows) > (1LL << 30)) return VSA_ERR_SHAPE;
   const float c2 = scale * kLog2e;
-#define VSA_F(DD, BB)                                                                        \
-  if (D == DD && be == BB) {                                                                 \
-    hipLaunchKernelGGL((sparse_fwd_f32m_kernel<DD, BB>), dim3((unsigned)tiles), dim3(128), 0, \
-                       s, (const float*)q, (const float*)k, (const float*)v, selected, kv_vbs, \
-                       (float*)out, (float*)fine, lse, (const float*)out_c,                \
-                       (const float*)gate, gate_mode, gate_heads, tph, (int)sq, (int)skv,     \
-                       (int)(sq / BB), (int)(skv / BB), topk, c2);                           \
-    return vsa_check_launch();                                                               \
+#define VSA_F(DD, BB)                                                                           \
+  if (D == DD && be == BB) {                                                                    \
+    if constexpr (DD <= 128) {                                                                  \
+      using C = SplitCfg<DD, BB>;                                                               \
+      const int tph = (int)(sq / C::ROWS), tiles = (int)(bh * tph);                             \
+      hipLaunchKernelGGL((sparse_fwd_f32_kernel<DD, BB>), dim3((unsigned)((tiles + 7) / 8 * 8)), \
+                         dim3(C::NT), 0, s, (const float*)q, (const float*)k, (const float*)v,  \
+                         selected, kv_vbs, (float*)out, (float*)fine, lse, (const float*)out_c, \
+                         (const float*)gate, gate_mode, gate_heads, tiles, tph, (int)sq,        \
+                         (int)skv, (int)(sq / BB), (int)(skv / BB), topk, c2);                  \
+    } else {                                                                                    \
+      const int tph = (int)(sq / kRows);                                                        \
+      hipLaunchKernelGGL((sparse_fwd_f32m_kernel<DD, BB>), dim3((unsigned)(bh * tph)),          \
+                         dim3(128), 0, s, (const float*)q, (const float*)k, (const float*)v,    \
+                         selected, kv_vbs, (float*)out, (float*)fine, lse, (const float*)out_c, \
+                         (const float*)gate, gate_mode, gate_heads, tph, (int)sq, (int)skv,     \
+                         (int)(sq / BB), (int)(skv / BB), topk, c2);                            \
+    }                                                                                           \
+    return vsa_check_launch();                                                                  \
   }
   VSA_F32_SHAPES(VSA_F)
 #undef VSA_F
@@ -600,18 +1090,27 @@ int sparse_dq_f32(const void* q, const void* k, const void* v, const void* dout,
                   int64_t bh, int64_t sq, int64_t skv, int D, int be, int topk, float scale,
                   hipStream_t s) {
   if (!f32_shape(D, be)) return VSA_ERR_UNSUPPORTED;
-  const int64_t tiles = bh * (sq / kRows);
-  if (tiles > (1LL << 30)) return VSA_ERR_SHAPE;
-  const int tph = (int)(sq / kRows);
+  if (bh * (sq / kRows) > (1LL << 30)) return VSA_ERR_SHAPE;
   const float c2 = scale * kLog2e;
-#define VSA_F(DD, BB)                                                                        \
-  if (D == DD && be == BB) {                                                                 \
-    hipLaunchKernelGGL((sparse_dq_f32m_kernel<DD, BB>), dim3((unsigned)tiles), dim3(128), 0, \
-                       s, (const float*)q, (const float*)k, (const float*)v,                 \
-                       (const float*)dout, lse, delta, selected, kv_vbs, (float*)dq,         \
-                       (const float*)dqc, q_vbs, tph, (int)sq, (int)skv, (int)(sq / BB),     \
-                       (int)(skv / BB), topk, c2, scale);                                    \
-    return vsa_check_launch();                                                               \
+#define VSA_F(DD, BB)                                                                           \
+  if (D == DD && be == BB) {                                                                    \
+    if constexpr (DD <= 128) {                                                                  \
+      using C = SplitCfg<DD, BB>;                                                               \
+      const int tph = (int)(sq / C::ROWS), tiles = (int)(bh * tph);                             \
+      hipLaunchKernelGGL((sparse_dq_f32_kernel<DD, BB>), dim3((unsigned)((tiles + 7) / 8 * 8)), \
+                         dim3(C::NT), 0, s, (const float*)q, (const float*)k, (const float*)v,  \
+                         (const float*)dout, lse, delta, selected, kv_vbs, (float*)dq,          \
+                         (const float*)dqc, q_vbs, tiles, tph, (int)sq, (int)skv,               \
+                         (int)(sq / BB), (int)(skv / BB), topk, c2, scale);                     \
+    } else {                                                                                    \
+      const int tph = (int)(sq / kRows);                                                        \
+      hipLaunchKernelGGL((sparse_dq_f32m_kernel<DD, BB>), dim3((unsigned)(bh * tph)),           \
+                         dim3(128), 0, s, (const float*)q, (const float*)k, (const float*)v,    \
+                         (const float*)dout, lse, delta, selected, kv_vbs, (float*)dq,          \
+                         (const float*)dqc, q_vbs, tph, (int)sq, (int)skv, (int)(sq / BB),      \
+                         (int)(skv / BB), topk, c2, scale);                                     \
+    }                                                                                           \
+    return vsa_check_launch();                                                                  \
   }
   VSA_F32_SHAPES(VSA_F)
 #undef VSA_F
@@ -624,30 +1123,29 @@ int sparse_dkdv_f32(const void* q, const void* k, const void* v, const void* dou
                     void* dk, void* dv, const void* dkc, const void* dvc, int64_t bh, int64_t sq,
                     int64_t skv, int D, int be, int topk, float scale, hipStream_t s) {
   if (!f32_shape(D, be)) return VSA_ERR_UNSUPPORTED;
-  const int64_t tiles = bh * (skv / kRows);
-  if (tiles > (1LL << 30)) return VSA_ERR_SHAPE;
-  const int tph = (int)(skv / kRows);
+  if (bh * (skv / kRows) > (1LL << 30)) return VSA_ERR_SHAPE;
   const float c2 = scale * kLog2e;
   // head_dim 64 / 128 on the matrix core, 256 on the vector ALU
-#define VSA_F(DD, BB)                                                                        \
-  if constexpr (DD <= 128) {                                                                 \
-  if (D == DD && be == BB) {                                                                 \
-    hipLaunchKernelGGL((sparse_dkdv_f32m_kernel<DD, BB>), dim3((unsigned)tiles), dim3(128), 0, \
-                       s, (const float*)q, (const float*)k, (const float*)v,                 \
-                       (const float*)dout, lse, delta, counts, offsets, inverse, kv_vbs,     \
-                       (float*)dk, (float*)dv, (const float*)dkc, (const float*)dvc, tph,    \
-                       (int)sq, (int)skv, (int)(sq / BB), (int)(skv / BB), topk, c2, scale); \
-    return vsa_check_launch();                                                               \
-  }                                                                                          \
-  } else {                                                                                   \
-  if (D == DD && be == BB) {                                                                 \
-    hipLaunchKernelGGL((sparse_dkdv_f32_kernel<DD, BB>), dim3((unsigned)tiles), dim3(256), 0, \
-                       s, (const float*)q, (const float*)k, (const float*)v,                 \
-                       (const float*)dout, lse, delta, counts, offsets, inverse, kv_vbs,     \
-                       (float*)dk, (float*)dv, (const float*)dkc, (const float*)dvc, tph,    \
-                       (int)sq, (int)skv, (int)(sq / BB), (int)(skv / BB), topk, c2, scale); \
-    return vsa_check_launch();                                                               \
-  }                                                                                          \
+#define VSA_F(DD, BB)                                                                             \
+  if (D == DD && be == BB) {                                                                      \
+    if constexpr (DD <= 128) {                                                                    \
+      using C = SplitCfg<DD, BB>;                                                                 \
+      const int tph = (int)(skv / C::ROWS), tiles = (int)(bh * tph);                              \
+      hipLaunchKernelGGL((sparse_dkdv_f32_kernel<DD, BB>), dim3((unsigned)((tiles + 7) / 8 * 8)), \
+                         dim3(C::NT), 0, s, (const float*)q, (const float*)k, (const float*)v,    \
+                         (const float*)dout, lse, delta, counts, offsets, inverse, kv_vbs,        \
+                         (float*)dk, (float*)dv, (const float*)dkc, (const float*)dvc, tiles,     \
+                         tph, (int)sq, (int)skv, (int)(sq / BB), (int)(skv / BB), topk, c2,       \
+                         scale);                                                                  \
+    } else {                                                                                      \
+      const int tph = (int)(skv / kRows);                                                         \
+      hipLaunchKernelGGL((sparse_dkdv_f32v_kernel<DD, BB>), dim3((unsigned)(bh * tph)),           \
+                         dim3(256), 0, s, (const float*)q, (const float*)k, (const float*)v,      \
+                         (const float*)dout, lse, delta, counts, offsets, inverse, kv_vbs,        \
+                         (float*)dk, (float*)dv, (const float*)dkc, (const float*)dvc, tph,       \
+                         (int)sq, (int)skv, (int)(sq / BB), (int)(skv / BB), topk, c2, scale);    \
+    }                                                                                             \
+    return vsa_check_launch();                                                                    \
   }
   VSA_F32_SHAPES(VSA_F)
 #undef VSA_F

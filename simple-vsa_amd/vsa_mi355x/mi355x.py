@@ -19,8 +19,8 @@ The building blocks (pooling, coarse attention + Top-K, CSR inversion, fine
 forward / backward) are exposed as functions so tests can check each kernel.
 
 The kernels exist for block volumes 64 / 128 / 256 and head dims 64 / 128 /
-256; bf16 / fp16 run on the MFMA kernels, fp32 on fp32 vector-ALU kernels
-(no rounding below fp32 anywhere on its path).  Other shapes the reference accepts on the GPU (volume in [1, 128],
+256; bf16 / fp16 run on the MFMA kernels, fp32 on kernels of its own (no
+rounding below fp32 anywhere on its path).  Other shapes the reference accepts on the GPU (volume in [1, 128],
 head_dim <= 256; triton_impl.py:379-384) run on the same kernels after a
 differentiable zero-padding of each block to the next kernel volume and of
 the head dim to the next kernel width (gfx950 row kernels); the softmax scale
