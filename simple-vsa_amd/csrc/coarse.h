@@ -1,4 +1,4 @@
-// Host launchers of the MFMA coarse-attention kernels and the radix Top-K
+// Host launchers of the MFMA coarse-attention kernels and the Top-K route
 // (coarse.hip); the C ABI entry points in common.hip dispatch to them for the
 // shapes they cover.
 #pragma once
@@ -8,14 +8,15 @@
 
 namespace vsa {
 
-// bf16 / fp16 with head_dim 64 or 128
-bool coarse_mfma_supported(int D, int dtype);
+// bf16 / fp16 with head_dim 64 or 128 (the backward: 256 up to 768 key blocks too)
+bool coarse_fwd_mfma_supported(int D, int dtype);
+bool coarse_bwd_mfma_supported(int D, int kb, int dtype);
 
 int coarse_fwd_mfma(const void* qc, const void* kc, const void* vc, float* scores, float* probs,
                     void* outc, int64_t bh, int qb, int kb, int D, float scale, int dtype,
                     hipStream_t s);
 
-int topk_radix(const float* scores, int32_t* selected, int64_t rows, int kb, int topk,
+int topk_route(const float* scores, int32_t* selected, int64_t rows, int kb, int topk,
                hipStream_t s);
 
 int coarse_bwd_mfma(const void* qc, const void* kc, const void* vc, const float* probs,

@@ -166,12 +166,36 @@ constexpr int kMaxRouteBlocks = 16000;
 // batch * heads: the per-(batch, head) passes put it in the grid's y dimension
 constexpr int64_t kMaxGridY = 65535;
 static int max_coarse_blocks(int D, int dtype) {
-  return coarse_mfma_supported(D, dtype) ? kMaxRouteBlocks : kMaxCoarseBlocks;
+  return coarse_fwd_mfma_supported(D, dtype) ? kMaxRouteBlocks : kMaxCoarseBlocks;
+}
+
+// x . row in fp32, in ascending order of the dims whatever the loads' width (16
+// bytes, several in flight, where rows are 16-byte aligned): the order decides
+// near-ties of the route.
+template <typename T>
+__device__ __forceinline__ float dot_row(const float* x, const T* __restrict__ row, int D) {
+  constexpr int VEC = 16 / sizeof(T), UN = 8;
+  float dot = 0.f;
+  int d = 0;
+  if (D % VEC == 0) {
+    for (; d + UN * VEC <= D; d += UN * VEC) {
+      u32x4 raw[UN];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) raw[u] = *reinterpret_cast<const u32x4*>(row + d + u * VEC);
+#pragma unroll
+      for (int u = 0; u < UN; ++u)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          dot = fmaf(x[d + u * VEC + e], Elem<T>::to_f(reinterpret_cast<const T*>(&raw[u])[e]), dot);
+    }
+  }
+  for (; d < D; ++d) dot = fmaf(x[d], Elem<T>::to_f(row[d]), dot);
+  return dot;
 }
 
 // Generic coarse forward (fp32, or head dims the MFMA kernels do not take):
 // one workgroup per (bh, query block); scores in T, softmax in T, out_c in T
-// (common.py:159-166).  The Top-K route runs afterwards (topk_radix).
+// (common.py:159-166).  The Top-K route runs afterwards (topk_route).
 template <typename T>
 __global__ __launch_bounds__(256) void coarse_fwd_kernel(
     const T* __restrict__ qc, const T* __restrict__ kc, const T* __restrict__ vc,
@@ -190,9 +214,7 @@ __global__ __launch_bounds__(256) void coarse_fwd_kernel(
   const T* kbase = kc + b * kb * (int64_t)D;
   float lmax = -INFINITY;
   for (int j = threadIdx.x; j < kb; j += 256) {
-    const T* kr = kbase + (int64_t)j * D;
-    float dot = 0.f;
-    for (int d = 0; d < D; ++d) dot = fmaf(qrow[d], Elem<T>::to_f(kr[d]), dot);
+    const float dot = dot_row(qrow, kbase + (int64_t)j * D, D);
     const float s = round_t<T>(round_t<T>(dot) * scale);
     srow[j] = s;
     lmax = fmaxf(lmax, s);
@@ -216,6 +238,7 @@ __global__ __launch_bounds__(256) void coarse_fwd_kernel(
   const T* vbase = vc + b * kb * (int64_t)D;
   for (int d = threadIdx.x; d < D; d += 256) {
     float acc = 0.f;
+#pragma unroll 16
     for (int j = 0; j < kb; ++j) acc = fmaf(prow[j], Elem<T>::to_f(vbase[(int64_t)j * D + d]), acc);
     outc[(b * qb + i) * D + d] = Elem<T>::from_f(acc);
   }
@@ -272,15 +295,37 @@ __global__ __launch_bounds__(kCsrNT) void csr_cols_kernel(const int32_t* __restr
   if (tid == 0) s_dup = 0;
   __syncthreads();
   int below = 0, dup = 0;
-  for (int e = tid; e < edges; e += kCsrNT) {
-    const int kv = sel[e];
-    if (kv < 0 || kv >= kb) continue;  // ids outside [0, kb) contribute nothing
-    if (kv < kv0) {
-      ++below;
-    } else if (kv < kv0 + nk) {
-      const int q = e / topk;
-      const uint32_t bit = 1u << (q & 31);
-      if (atomicOr(&cbits[(kv - kv0) * qw + (q >> 5)], bit) & bit) dup = 1;
+  // The scan is a chain of memory round trips: kUnroll edges' loads are in
+  // flight together, and an edge's query block follows from the one before
+  // (an integer division per edge took as long as the loads).  12 heads x 624
+  // blocks x topk 78: 57.7 -> 28.0 us.
+  constexpr int kUnroll = 8;
+  const int q_step = kCsrNT / topk, r_step = kCsrNT % topk;
+  int q = tid / topk, rem = tid % topk;  // edge e = q * topk + rem
+  for (int e0 = tid; e0 < edges; e0 += kUnroll * kCsrNT) {
+    int kvs[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int e = e0 + u * kCsrNT;
+      kvs[u] = e < edges ? sel[e] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int kv = kvs[u];
+      if (kv >= 0 && kv < kb) {  // ids outside [0, kb) contribute nothing
+        if (kv < kv0) {
+          ++below;
+        } else if (kv < kv0 + nk) {
+          const uint32_t bit = 1u << (q & 31);
+          if (atomicOr(&cbits[(kv - kv0) * qw + (q >> 5)], bit) & bit) dup = 1;
+        }
+      }
+      q += q_step;
+      rem += r_step;
+      if (rem >= topk) {
+        rem -= topk;
+        ++q;
+      }
     }
   }
   below = wave_incl_sum(below);
@@ -691,9 +736,7 @@ __global__ __launch_bounds__(256) void coarse_bwd_rows_kernel(
   const float* prow = probs + rowq * kb;
   float lsum = 0.f;
   for (int j = threadIdx.x; j < kb; j += 256) {
-    const T* vr = vbase + (int64_t)j * D;
-    float dot = 0.f;
-    for (int d = 0; d < D; ++d) dot = fmaf(grow[d], Elem<T>::to_f(vr[d]), dot);
+    const float dot = dot_row(grow, vbase + (int64_t)j * D, D);
     const float dp = round_t<T>(dot);
     dsrow[j] = dp;
     lsum = fmaf(prow[j], dp, lsum);
@@ -709,6 +752,7 @@ __global__ __launch_bounds__(256) void coarse_bwd_rows_kernel(
   const T* kbase = kc + b * kb * (int64_t)D;
   for (int d = threadIdx.x; d < D; d += 256) {
     float acc = 0.f;
+#pragma unroll 16
     for (int j = 0; j < kb; ++j) acc = fmaf(dsrow[j], Elem<T>::to_f(kbase[(int64_t)j * D + d]), acc);
     d_qc[rowq * D + d] = Elem<T>::from_f(acc);
   }
@@ -727,6 +771,7 @@ __global__ __launch_bounds__(256) void coarse_bwd_cols_kernel(
   const float* pb = probs + b * qb * (int64_t)kb;
   for (int d = threadIdx.x; d < D; d += 256) {
     float ak = 0.f, av = 0.f;
+#pragma unroll 8
     for (int i = 0; i < qb; ++i) {
       ak = fmaf(dsb[(int64_t)i * kb + j], Elem<T>::to_f(qbase[(int64_t)i * D + d]), ak);
       av = fmaf(pb[(int64_t)i * kb + j], Elem<T>::to_f(gbase[(int64_t)i * D + d]), av);
@@ -875,11 +920,11 @@ extern "C" int vsa_coarse_fwd(const void* q_c, const void* k_c, const void* v_c,
     return VSA_ERR_SHAPE;
   if (selected && (topk < 1 || topk > kb)) return VSA_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  if (coarse_mfma_supported(D, dtype)) {
+  if (coarse_fwd_mfma_supported(D, dtype)) {
     const int rc = coarse_fwd_mfma(q_c, k_c, v_c, scores, probs, out_c, bh, qb, kb, D, scale,
                                    dtype, s);
     if (rc || !selected) return rc;
-    return topk_radix(scores, selected, bh * qb, kb, topk, s);
+    return topk_route(scores, selected, bh * qb, kb, topk, s);
   }
   const size_t shm = (size_t)(D + 2 * kb + 4) * sizeof(float);
   VSA_DISPATCH_ALL(dtype, T, {
@@ -889,7 +934,7 @@ extern "C" int vsa_coarse_fwd(const void* q_c, const void* k_c, const void* v_c,
   });
   const int rc = vsa_check_launch();
   if (rc || !selected) return rc;
-  return topk_radix(scores, selected, bh * qb, kb, topk, s);
+  return topk_route(scores, selected, bh * qb, kb, topk, s);
 }
 
 extern "C" int vsa_topk(const float* scores, int32_t* selected, int64_t rows, int32_t kb,
@@ -897,7 +942,7 @@ extern "C" int vsa_topk(const float* scores, int32_t* selected, int64_t rows, in
   if (!scores || !selected) return VSA_ERR_NULL;
   if (!vsa_aligned<16>(scores) || !vsa_aligned<4>(selected)) return VSA_ERR_ALIGN;
   if (rows <= 0 || kb <= 0 || kb > kMaxRouteBlocks || topk < 1 || topk > kb) return VSA_ERR_SHAPE;
-  return topk_radix(scores, selected, rows, kb, topk, (hipStream_t)stream);
+  return topk_route(scores, selected, rows, kb, topk, (hipStream_t)stream);
 }
 
 constexpr int kMaxCsrBlocks = 16000;  // Qb: a column of 500 words, 28 columns per workgroup
@@ -1017,7 +1062,7 @@ extern "C" int vsa_coarse_bwd(const void* q_c, const void* k_c, const void* v_c,
       D <= 0 || D > 1024)
     return VSA_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  if (coarse_mfma_supported(D, dtype))
+  if (coarse_bwd_mfma_supported(D, kb, dtype))
     return coarse_bwd_mfma(q_c, k_c, v_c, probs, d_out_c, ds, d_q_c, d_k_c, d_v_c, bh, qb, kb, D,
                            scale, dtype, s);
   const size_t shm = (size_t)(D + kb + 4) * sizeof(float);
