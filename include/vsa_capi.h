@@ -416,6 +416,41 @@ int vsa_sparse_bwd_dkdv_tiled(const void* q, const void* k, const void* v, const
                               int32_t head_dim, int32_t block_elements, int32_t topk, float scale,
                               int32_t* tile_order, int32_t dtype, void* stream);
 
+/*
+ * One whole forward or backward pass of an op, launched by one call: the
+ * sequence of the entry points above that the op consists of, on buffers carved
+ * from two workspaces (the caller's calls would each cost more host time than
+ * a small pass runs).  Replaces _vsa_with_sparse_executor and the autograd of
+ * its parts (triton_impl.py:1655-1731, 1530-1580) for
+ *  - the full op: `selected` NULL, q [BH, Sq, D] and k, v [BH, Skv, D];
+ *  - the fine branch on a caller's route: `selected` [BH, Qb, topk], no gate;
+ *  - the full op on raster-order tokens: `slot_rows` given (with s_out and heads
+ *    as in vsa_tile_pool_qkv), sq = skv = nb * block.
+ * A block volume or head dim without a kernel of its own runs zero-padded to
+ * kernel_block / kernel_dim (block in [1, kernel_block], not for raster
+ * tokens): q, k, v, gate, out and the gradients keep the caller's shapes.
+ */
+typedef struct vsa_op {
+  const void *q, *k, *v, *gate;
+  const int32_t *selected, *kv_vbs, *q_vbs, *slot_rows;
+  int64_t bh, sq, skv, s_out;
+  int32_t heads, head_dim, block, kernel_dim, kernel_block, topk, gate_mode, gate_heads, dtype;
+  int32_t keep;              /* the forward keeps what vsa_op_bwd needs in `saved` */
+  float scale;
+} vsa_op;
+
+/* Bytes of `saved` and of each pass's `scratch`, from the op's sizes and from
+ * which of its pointers are NULL. */
+int vsa_op_sizes(const vsa_op* op, int64_t* saved, int64_t* scratch_fwd, int64_t* scratch_bwd);
+
+int vsa_op_fwd(const vsa_op* op, void* out, void* saved, void* scratch, void* stream);
+
+/* `out`: the forward's result (the route op's delta needs it; else unused).  q,
+ * k, v and gate may be NULL where the forward kept copies (padded shapes; q, k,
+ * v of raster tokens), but a gate must then be announced by gate_mode. */
+int vsa_op_bwd(const vsa_op* op, const void* out, const void* dout, void* saved, void* scratch,
+               void* dq, void* dk, void* dv, void* d_gate, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

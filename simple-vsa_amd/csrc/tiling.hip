@@ -184,6 +184,67 @@ static bool row_grid(int64_t rows, int tpr_log2, int64_t batch, dim3& grid) {
   return true;
 }
 
+// ---------------------------------------------------------------------------
+// Blocks of `be` rows to blocks of `kbe` (PAD: rows and row ends added as zeros)
+// and back, for up to four tensors in one launch: a workgroup moves 32 rows of
+// one tensor's result, in units of 16 bytes where both row lengths allow.
+// Bound by HBM; a launch replaces four per tensor of the indexed moves
+// (rows_move_kernel and three for the zeros).
+// ---------------------------------------------------------------------------
+template <bool PAD, typename U>
+__device__ __forceinline__ void block_move_rows(const BlockMove& m, int y) {
+  const int be = m.be, kbe = m.kbe;
+  const int from = m.src_bytes[y] / (int)sizeof(U), to = m.dst_bytes[y] / (int)sizeof(U);
+  const int per = PAD ? kbe : be;  // rows of a block of the result
+  const int64_t row0 = (int64_t)blockIdx.x * 32;
+  const int64_t n0 = row0 / per;
+  const int t0 = (int)(row0 - n0 * per);
+  const int rows = (int)min((int64_t)32, m.rows[y] - row0);
+  const U* src = static_cast<const U*>(m.src[y]);
+  U* dst = static_cast<U*>(m.dst[y]) + row0 * to;
+  for (int x = threadIdx.x; x < rows * to; x += 256) {
+    const int r = x / to, u = x - r * to;
+    const int step = (t0 + r) / per, t = t0 + r - step * per;
+    U v = U{};
+    if (!PAD || (t < be && u < from)) v = src[((n0 + step) * (PAD ? be : kbe) + t) * from + u];
+    dst[x] = v;
+  }
+}
+
+template <bool PAD>
+__global__ __launch_bounds__(256) void block_move_kernel(BlockMove m) {
+  const int y = blockIdx.y;
+  if ((int64_t)blockIdx.x * 32 >= m.rows[y]) return;
+  switch (m.unit[y]) {
+    case 16: return block_move_rows<PAD, u32x4_t>(m, y);
+    case 8: return block_move_rows<PAD, u32x2_t>(m, y);
+    case 4: return block_move_rows<PAD, uint32_t>(m, y);
+    default: return block_move_rows<PAD, uint16_t>(m, y);
+  }
+}
+
+int block_move(BlockMove& m, bool pad, hipStream_t s) {
+  int64_t most = 0;
+  for (int i = 0; i < m.n; ++i) {
+    m.unit[i] = 2;
+    for (int u = 16; u > 2; u >>= 1)
+      if (m.src_bytes[i] % u == 0 && m.dst_bytes[i] % u == 0) {
+        m.unit[i] = u;
+        break;
+      }
+    if (m.rows[i] > most) most = m.rows[i];
+  }
+  const int64_t groups = (most + 31) / 32;
+  if (groups <= 0) return VSA_OK;
+  if (groups > (1LL << 31) - 1) return VSA_ERR_SHAPE;
+  const dim3 grid((unsigned)groups, (unsigned)m.n);
+  if (pad)
+    hipLaunchKernelGGL((block_move_kernel<true>), grid, dim3(256), 0, s, m);
+  else
+    hipLaunchKernelGGL((block_move_kernel<false>), grid, dim3(256), 0, s, m);
+  return vsa_check_launch();
+}
+
 }  // namespace vsa
 
 using namespace vsa;

@@ -74,6 +74,17 @@ int combine_f32gate(const void* fine, const void* out_c, const void* gate, int g
 // The shape checks combine_f32gate makes, for callers that must reject a call
 // before launching anything else.
 bool combine_f32gate_shape_ok(int64_t bh, int64_t sq, int D, int be, int dtype);
+// Up to four tensors whose blocks of be rows become blocks of kbe rows, or back
+// (block_move, tiling.hip): rows of the result, bytes of a source and a result
+// row.
+struct BlockMove {
+  const void* src[4];
+  void* dst[4];
+  int64_t rows[4];
+  int src_bytes[4], dst_bytes[4], unit[4];
+  int n, be, kbe;
+};
+int block_move(BlockMove& m, bool pad, hipStream_t s);
 // Scheduling counters (take_entry) of the persistent forward and dQ kernels for
 // launches on stream s, from a file-scope device array (common.hip): one slot
 // of zeroed counters per (device, stream), which every launch leaves zeroed.

@@ -49,6 +49,10 @@ SIGNATURES = {
     "vsa_rows_move": [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _P, _I64, _P,
                       _I64, _P],
     "vsa_rows_zero_unmarked": [_P, _I64, _I64, _I64, _P, _I64, _P, _P],
+    # a whole pass per call
+    "vsa_op_sizes": [_P, _P, _P, _P],
+    "vsa_op_fwd": [_P, _P, _P, _P, _P],
+    "vsa_op_bwd": [_P] * 10,
     # tiled sequences (tile / untile fused into the op)
     "vsa_tile_slot_rows": [_I32, _I32, _I32, _I32, _I32, _I32, _P, _P],
     "vsa_tile_pool_qkv": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I32,
@@ -64,6 +68,18 @@ SIGNATURES = {
                                   _P],
 }
 _RESTYPES = {"vsa_status_string": ctypes.c_char_p, "vsa_version": ctypes.c_char_p}
+
+
+class VsaOp(ctypes.Structure):
+    """``struct vsa_op`` of the header."""
+    _fields_ = ([(n, _P) for n in ("q", "k", "v", "gate", "selected", "kv_vbs", "q_vbs",
+                                   "slot_rows")]
+                + [(n, _I64) for n in ("bh", "sq", "skv", "s_out")]
+                + [(n, _I32) for n in ("heads", "head_dim", "block", "kernel_dim",
+                                       "kernel_block", "topk", "gate_mode", "gate_heads",
+                                       "dtype", "keep")]
+                + [("scale", _F)])
+
 
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None

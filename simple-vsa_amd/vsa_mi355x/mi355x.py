@@ -10,23 +10,26 @@ Public entry points keep the reference's operator API:
   block_size, sm_scale=None)`` -- drop-in for ``triton_sparse_attention``
   (triton_impl.py:1626-1652).
 
-Both are differentiable (one ``torch.autograd.Function`` each).  Every
-compute step is a HIP kernel behind ``_lib``; the host only validates,
-allocates outputs/workspace with ``torch.empty`` and launches on the current
-stream, with no device synchronisation.
+Both are differentiable (one ``torch.autograd.Function``).  Every compute step
+is a HIP kernel behind ``_lib``; the host only validates, allocates outputs /
+workspace with ``torch.empty`` and launches on the current stream, with no
+device synchronisation.
 
 The building blocks (pooling, coarse attention + Top-K, CSR inversion, fine
 forward / backward) are exposed as functions so tests can check each kernel.
 
 The kernels exist for block volumes 64 / 128 / 256 and head dims 64 / 128 /
 256; bf16 / fp16 run on the MFMA kernels, fp32 on kernels of its own (no
-rounding below fp32 anywhere on its path).  Other shapes the reference accepts on the GPU (volume in [1, 128],
-head_dim <= 256; triton_impl.py:379-384) run on the same kernels after a
-differentiable zero-padding of each block to the next kernel volume and of
-the head dim to the next kernel width (gfx950 row kernels); the softmax scale
-stays 1/sqrt(head_dim) of the caller's tensors.  Padded query rows are
-computed and dropped, padded keys are masked by the block sizes, padded
-channels are zero in every dot product.
+rounding below fp32 anywhere on its path).  Other shapes the reference accepts
+on the GPU (volume in [1, 128], head_dim <= 256; triton_impl.py:379-384) run on
+the same kernels after zero-padding each block to the next kernel volume and
+the head dim to the next kernel width; the softmax scale stays 1/sqrt(head_dim)
+of the caller's tensors.  Padded query rows are computed and dropped, padded
+keys are masked by the block sizes, padded channels are zero in every dot
+product.
+
+Both ops run a whole pass as one call into the library (``launch``); the
+functions here check, convert and pick the op's sizes.
 """
 
 from __future__ import annotations
@@ -39,7 +42,7 @@ import torch
 from torch import Tensor
 from torch.autograd.function import once_differentiable
 
-from . import _lib
+from . import _lib, launch
 from .tiling import _move, _zero_unmarked
 
 SUPPORTED_BLOCKS = (64, 128, 256)
@@ -196,6 +199,11 @@ class _Unpad(torch.autograd.Function):
         return _Pad.apply(g, rows, *ctx.padded), None, None
 
 
+def _padded_shape(q, be) -> bool:
+    """No kernel of its own for this block volume and head dim."""
+    return _kernel_block(be) != be or _kernel_dim(q.shape[-1]) != q.shape[-1]
+
+
 def _padded(q, k, be):
     """(kbe, kd, pad_q, pad_k, unpad_out) for a shape without its own kernel,
     or None when the kernels take the tensors as they are."""
@@ -240,6 +248,8 @@ def _empty_batch(q: Tensor, *others: Optional[Tensor]) -> Tensor:
 
 
 def _i32(x: Tensor, device) -> Tensor:
+    if x.dtype is torch.int32 and x.device == device and x.is_contiguous():
+        return x
     return x.to(device=device, dtype=torch.int32).contiguous()
 
 
@@ -434,24 +444,11 @@ def dkdv_tile_order(counts, bh, skv, head_dim, block_elements):
 # Explicit-route executor (triton_impl.py:1530-1652)
 # ---------------------------------------------------------------------------
 
-class _SparseAttention(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, selected, vbs, block_elements, scale):
-        out, lse, _ = sparse_forward(q, k, v, selected, vbs, block_elements, scale,
-                                     want_lse=True)
-        ctx.save_for_backward(q, k, v, out, lse, selected, vbs)
-        ctx.block_elements, ctx.scale = block_elements, scale
-        return out
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, dout):
-        q, k, v, out, lse, selected, vbs = ctx.saved_tensors
-        dout = _aligned16(dout.contiguous())
-        delta, _, _ = backward_prep(out, dout, ctx.block_elements)
-        dq, dk, dv = sparse_backward(q, k, v, dout, lse, delta, selected, vbs,
-                                     ctx.block_elements, ctx.scale)
-        return dq, dk, dv, None, None, None, None
+def _spec(q, k, gate, be, topk, scale, route=False) -> launch.Spec:
+    """The op on head-major [B, H, S, D] tensors."""
+    b, h, sq, d = q.shape
+    return launch.Spec(b * h, sq, k.shape[2], 0, 0, d, be, _kernel_dim(d), _kernel_block(be), topk,
+                   _gate_mode(gate, d, q.dtype), h, _lib.dtype_code(q.dtype), 0, scale, route)
 
 
 def _validate_route(q, k, selected, variable_block_sizes, be):
@@ -481,21 +478,11 @@ def mi355x_sparse_attention(q: Tensor, k: Tensor, v: Tensor, selected: Tensor,
     if q.shape[0] * q.shape[1] == 0:
         return _empty_batch(q, k, v)
     scale = sm_scale if sm_scale is not None else 1.0 / math.sqrt(q.shape[-1])
-    pads = _padded(q, k, be)
-    if pads is not None:
-        kbe, _, pad_q, pad_k, unpad_out = pads
-        with torch.cuda.device(q.device):
-            out = mi355x_sparse_attention(pad_q(q), pad_k(k), pad_k(v), selected,
-                                          variable_block_sizes, block_size=(1, 1, kbe),
-                                          sm_scale=scale)
-            return unpad_out(out)
     q, k, v = (_aligned16(x.contiguous()) for x in (q, k, v))
     selected = _i32(selected, q.device)
     vbs = _i32(variable_block_sizes, q.device)
-    with torch.cuda.device(q.device):
-        if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
-            return _SparseAttention.apply(q, k, v, selected, vbs, be, float(scale))
-        return sparse_forward(q, k, v, selected, vbs, be, scale, want_lse=False)[0]
+    return launch.run(_spec(q, k, None, be, selected.shape[-1], float(scale), route=True), q, k, v,
+                  None, selected, vbs, None, None)
 
 
 def mi355x_sparse_executor(block_size):
@@ -518,14 +505,15 @@ def mi355x_sparse_executor(block_size):
 # ---------------------------------------------------------------------------
 
 class _VSA(torch.autograd.Function):
+    """The op step by step, for ``return_aux`` (its intermediates are tensors)."""
+
     @staticmethod
-    def forward(ctx, q, k, v, gate, vbs, qvbs, topk_, be, scale, aux=None):
+    def forward(ctx, q, k, v, gate, vbs, qvbs, topk_, be, scale, aux):
         qc, kc, vc = block_mean_qkv(q, k, v, vbs, qvbs, be)
         scores, probs, outc, sel = coarse_forward(qc, kc, vc, topk_, scale)
         out, lse, fine = sparse_forward(q, k, v, sel, vbs, be, scale, out_c=outc, gate=gate,
                                         want_lse=True)
-        if aux is not None:
-            aux.update(scores=scores, selected=sel, out_c=outc, fine=fine)
+        aux.update(scores=scores, selected=sel, out_c=outc, fine=fine)
         ctx.save_for_backward(q, k, v, gate, vbs, qvbs, qc, kc, vc, probs, outc, sel, fine, lse)
         ctx.be, ctx.scale = be, scale
         return out
@@ -540,6 +528,16 @@ class _VSA(torch.autograd.Function):
         dq, dk, dv = sparse_backward(q, k, v, dout, lse, delta, sel, vbs, ctx.be, ctx.scale,
                                      dqc=dqc, dkc=dkc, dvc=dvc, q_variable_block_sizes=qvbs)
         return dq, dk, dv, d_gate, None, None, None, None, None, None
+
+
+def _broadcasts(gate: Tensor, q: Tensor) -> bool:
+    """The gate's shape broadcasts to q's."""
+    if gate.ndim == 4 and gate.shape[:3] == q.shape[:3] and gate.shape[3] in (1, q.shape[3]):
+        return True   # the usual ones, without torch's general rule (25 us)
+    try:
+        return torch.broadcast_shapes(gate.shape, q.shape) == q.shape
+    except RuntimeError:
+        return False
 
 
 def _prepare_gate(gate: Optional[Tensor], q: Tensor) -> Optional[Tensor]:
@@ -557,11 +555,7 @@ def _prepare_gate(gate: Optional[Tensor], q: Tensor) -> Optional[Tensor]:
     if gate is None:
         return None
     b, h, s, d = q.shape
-    try:
-        ok = torch.broadcast_shapes(gate.shape, q.shape) == q.shape
-    except RuntimeError:
-        ok = False
-    if not ok:
+    if not _broadcasts(gate, q):
         raise ValueError("compress_attn_weight must have the same shape as q, or a shape that "
                          "broadcasts to it (e.g. [batch, heads, seq_len, 1])")
     gate = gate.to(device=q.device)
@@ -608,25 +602,29 @@ def mi355x_vsa(q: Tensor, k: Tensor, v: Tensor, variable_block_sizes: Tensor,
     scale = float(sm_scale) if sm_scale is not None else 1.0 / math.sqrt(q.shape[-1])
     vbs = _i32(variable_block_sizes, q.device)
     qvbs = _i32(q_variable_block_sizes, q.device)
-    aux = {} if return_aux else None
-    with torch.cuda.device(q.device):
-        if aux is None and _raster_views(q, k, v, gate, be):
+    if not return_aux:
+        if _raster_views(q, k, v, gate, be):
             from . import tiled
             return tiled.vsa_token_major_views(q, k, v, gate, vbs, qvbs, topk, be, scale)
+        if gate is not None and not gate.is_contiguous() and _padded_shape(q, be):
+            gate = gate.contiguous()   # a token-major gate: the padded copies are head-major
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        return launch.run(_spec(q, k, gate, be, topk, scale), q, k, v, gate, None, vbs, qvbs, None)
+    aux = {}
+    with torch.cuda.device(q.device):
         pads = _padded(q, k, be)
         if pads is not None:
             kbe, kd, pad_q, pad_k, unpad_out = pads
             gate = pad_q(gate, kd if gate is not None and gate.shape[-1] == q.shape[-1] else 1)
             out = unpad_out(_vsa(pad_q(q), pad_k(k), pad_k(v), gate, vbs, qvbs, topk, kbe,
                                  scale, aux))
-            if aux is not None:
-                aux["fine"] = _unpad(aux["fine"], _block_rows(q.shape[2], be, kbe, q.device),
-                                     tuple(q.shape))
-                aux["out_c"] = aux["out_c"][..., :q.shape[-1]]
+            aux["fine"] = _unpad(aux["fine"], _block_rows(q.shape[2], be, kbe, q.device),
+                                 tuple(q.shape))
+            aux["out_c"] = aux["out_c"][..., :q.shape[-1]]
         else:
             out = _vsa(q.contiguous(), k.contiguous(), v.contiguous(), gate, vbs, qvbs, topk,
                        be, scale, aux)
-    return (out, _aux_dict(aux, q, be)) if return_aux else out
+    return out, _aux_dict(aux, q, be)
 
 
 def _aux_dict(aux: dict, q: Tensor, be: int) -> dict:
@@ -652,10 +650,10 @@ def _empty_aux(q: Tensor, k: Tensor, be: int) -> dict:
             "out_compress": q.new_empty(q.shape), "out_sparse": q.new_empty(q.shape)}
 
 
-def _vsa(q, k, v, gate, vbs, qvbs, topk, be, scale, aux=None):
-    """The op on kernel-native shapes (contiguous, be and head dim supported).
-    With ``aux`` (a dict) the forward's scores, route, ``out_c`` and fine output
-    are put into it."""
+def _vsa(q, k, v, gate, vbs, qvbs, topk, be, scale, aux):
+    """The op step by step on kernel-native shapes (contiguous, be and head dim
+    supported); the forward's scores, route, ``out_c`` and fine output are put
+    into the dict ``aux``."""
     needs_grad = torch.is_grad_enabled() and (
         q.requires_grad or k.requires_grad or v.requires_grad
         or (gate is not None and gate.requires_grad))
@@ -664,9 +662,8 @@ def _vsa(q, k, v, gate, vbs, qvbs, topk, be, scale, aux=None):
     qc, kc, vc = block_mean_qkv(q, k, v, vbs, qvbs, be)
     scores, _, outc, sel = coarse_forward(qc, kc, vc, topk, scale)
     out, _, fine = sparse_forward(q, k, v, sel, vbs, be, scale, out_c=outc, gate=gate,
-                                  want_lse=False, want_fine=aux is not None)
-    if aux is not None:
-        aux.update(scores=scores, selected=sel, out_c=outc, fine=fine)
+                                  want_lse=False, want_fine=True)
+    aux.update(scores=scores, selected=sel, out_c=outc, fine=fine)
     return out
 
 

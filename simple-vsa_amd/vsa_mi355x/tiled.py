@@ -32,9 +32,8 @@ from typing import Optional, Tuple
 
 import torch
 from torch import Tensor
-from torch.autograd.function import once_differentiable
 
-from . import _lib
+from . import _lib, launch
 from . import mi355x as M
 from . import tiling
 
@@ -73,78 +72,14 @@ def _dims(x, token_major):
     return tuple(x.shape)
 
 
-def _tile_pool(q, k, v, rows, qvbs, vbs, nb, be, token_major):
+def _spec(q, gate, topk, nb, be, scale, token_major) -> launch.Spec:
+    """The op on raster-order tokens (slot table of nb * be rows)."""
     b, h, s_out, d = _dims(q, token_major)
-    tiled = (b, h, nb * be, d)
-    qt, kt, vt = (torch.empty(tiled, device=q.device, dtype=q.dtype) for _ in range(3))
-    qc, kc, vc = (torch.empty((b, h, nb, d), device=q.device, dtype=q.dtype) for _ in range(3))
-    _lib.call("vsa_tile_pool_qkv", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(rows),
-              _lib.ptr(qvbs), _lib.ptr(vbs), _lib.ptr(qt), _lib.ptr(kt), _lib.ptr(vt), _lib.ptr(qc),
-              _lib.ptr(kc), _lib.ptr(vc), b * h, s_out, h if token_major else 0, nb, d, be,
-              _lib.dtype_code(q.dtype), _lib.stream_of(q))
-    return qt, kt, vt, qc, kc, vc
-
-
-def _forward(q, k, v, gate, rows, vbs, qvbs, topk, nb, be, scale, want_lse, token_major):
-    b, h, s_out, d = _dims(q, token_major)
-    qt, kt, vt, qc, kc, vc = _tile_pool(q, k, v, rows, qvbs, vbs, nb, be, token_major)
-    _, probs, outc, sel = M.coarse_forward(qc, kc, vc, topk, scale)
-    L = nb * be
-    out = torch.empty_like(q)
-    lse = torch.empty((b, h, L), device=q.device, dtype=torch.float32) if want_lse else None
-    fine = torch.empty_like(qt) if want_lse else None
-    gmode = M._gate_mode(gate, d, q.dtype)
-    _lib.call("vsa_sparse_fwd_tiled", _lib.ptr(qt), _lib.ptr(kt), _lib.ptr(vt), _lib.ptr(sel),
-              _lib.ptr(vbs), _lib.ptr(out), _lib.ptr(fine), _lib.ptr(lse), _lib.ptr(outc),
-              _lib.ptr(gate), gmode, _lib.ptr(rows), s_out, h if token_major else 0, b * h, L, L,
-              d, be, topk, float(scale), _lib.dtype_code(q.dtype), _lib.stream_of(q))
-    return out, (qt, kt, vt, qc, kc, vc, probs, outc, sel, fine, lse)
-
-
-class _VSATiled(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, gate, rows, vbs, qvbs, topk_, nb, be, scale, token_major):
-        out, saved = _forward(q, k, v, gate, rows, vbs, qvbs, topk_, nb, be, scale, True,
-                              token_major)
-        ctx.save_for_backward(gate, rows, vbs, qvbs, *saved)
-        ctx.dims = (q.shape, _dims(q, token_major), nb, be, scale, token_major)
-        return out
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, dout):
-        gate, rows, vbs, qvbs, qt, kt, vt, qc, kc, vc, probs, outc, sel, fine, lse = \
-            ctx.saved_tensors
-        shape, (b, h, s_out, d), nb, be, scale, token_major = ctx.dims
-        heads = h if token_major else 0
-        L = nb * be
-        dout = M._aligned16(dout.contiguous())
-        code, stream = _lib.dtype_code(dout.dtype), _lib.stream_of(dout)
-        delta = torch.empty((b, h, L), device=dout.device, dtype=torch.float32)
-        d_outc = torch.empty_like(outc)
-        d_gate = torch.empty_like(gate) if gate is not None else None
-        dout_t = torch.empty_like(qt)
-        gmode = M._gate_mode(gate, d, dout.dtype)
-        _lib.call("vsa_bwd_prep_tiled", _lib.ptr(fine), _lib.ptr(dout), _lib.ptr(outc),
-                  _lib.ptr(gate), gmode, _lib.ptr(rows), s_out, heads, _lib.ptr(delta),
-                  _lib.ptr(d_outc), _lib.ptr(d_gate), _lib.ptr(dout_t), b * h, L, d, be, code,
-                  stream)
-        dqc, dkc, dvc = M.coarse_backward(qc, kc, vc, probs, d_outc, scale)
-        tk = sel.shape[-1]
-        dq = torch.empty(shape, device=dout.device, dtype=dout.dtype)
-        dk, dv = torch.empty_like(dq), torch.empty_like(dq)
-        _lib.call("vsa_sparse_bwd_dq_tiled", _lib.ptr(qt), _lib.ptr(kt), _lib.ptr(vt),
-                  _lib.ptr(dout_t), _lib.ptr(lse), _lib.ptr(delta), _lib.ptr(sel), _lib.ptr(vbs),
-                  _lib.ptr(dq), _lib.ptr(dqc), _lib.ptr(qvbs), _lib.ptr(rows), s_out, heads, b * h,
-                  L, L, d, be, tk, float(scale), code, stream)
-        inverse, offsets, counts = M.invert_routes(sel, nb)
-        order = M.dkdv_tile_order(counts, b * h, L, d, be)
-        _lib.call("vsa_sparse_bwd_dkdv_tiled", _lib.ptr(qt), _lib.ptr(kt), _lib.ptr(vt),
-                  _lib.ptr(dout_t), _lib.ptr(lse), _lib.ptr(delta), _lib.ptr(counts),
-                  _lib.ptr(offsets), _lib.ptr(inverse), _lib.ptr(vbs), _lib.ptr(dk), _lib.ptr(dv),
-                  _lib.ptr(dkc), _lib.ptr(dvc), _lib.ptr(rows), s_out, heads, b * h, L, L, d, be,
-                  tk, float(scale), _lib.ptr(order), code, stream)
-        return dq, dk, dv, d_gate, None, None, None, None, None, None, None, None
+    # a gate is [.., S, D] or [.., S, 1] in the raster tensors' own layout
+    mode = (_lib.GATE_NONE if gate is None else
+            _lib.GATE_PER_TOKEN if gate.shape[-1] == 1 else _lib.GATE_FULL)
+    return launch.Spec(b * h, nb * be, nb * be, s_out, h if token_major else 0, d, be, d, be, topk,
+                   mode, 0, _lib.dtype_code(q.dtype), 0, scale, False)
 
 
 @functools.lru_cache(maxsize=16)
@@ -165,15 +100,8 @@ def vsa_token_major_views(q, k, v, gate, vbs, qvbs, topk, be, scale):
     g = None if gate is None else gate.transpose(1, 2).contiguous()
     s = qr.shape[1]
     rows = _identity_rows(s, q.device)
-    needs_grad = torch.is_grad_enabled() and (
-        q.requires_grad or k.requires_grad or v.requires_grad
-        or (g is not None and g.requires_grad))
-    if needs_grad:
-        out = _VSATiled.apply(qr, kr, vr, g, rows, vbs, qvbs, topk, s // be, be, scale, True)
-    else:
-        out = _forward(qr, kr, vr, g, rows, vbs, qvbs, topk, s // be, be, scale, False,
-                       True)[0]
-    return out.transpose(1, 2)
+    return launch.run(_spec(qr, g, topk, s // be, be, scale, True), qr, kr, vr, g, None, vbs, qvbs,
+                  rows).transpose(1, 2)
 
 
 def _composition(q, k, v, meta, nb, be, tile_size, topk, gate, token_major=False):
@@ -227,11 +155,7 @@ def mi355x_vsa_tiled(q: Tensor, k: Tensor, v: Tensor, dit_seq_shape: Tuple[int, 
     if seq != s_out:
         raise ValueError(f"seq_len {seq} is not T*H*W = {s_out} of dit_seq_shape {shape}")
     if compress_attn_weight is not None:
-        try:
-            ok = torch.broadcast_shapes(compress_attn_weight.shape, q.shape) == q.shape
-        except RuntimeError:
-            ok = False
-        if not ok:
+        if not M._broadcasts(compress_attn_weight, q):
             raise ValueError("compress_attn_weight must have the same shape as q, or a shape "
                              "that broadcasts to it (e.g. [batch, heads, seq_len, 1])")
     be = math.prod(ts)
@@ -258,12 +182,5 @@ def mi355x_vsa_tiled(q: Tensor, k: Tensor, v: Tensor, dit_seq_shape: Tuple[int, 
         q, k, v = (M._aligned16(x.contiguous()) for x in (q, k, v))
         if gate is not None:
             gate = M._aligned16(gate.contiguous())
-        scale = 1.0 / math.sqrt(d)
-        needs_grad = torch.is_grad_enabled() and (
-            q.requires_grad or k.requires_grad or v.requires_grad
-            or (gate is not None and gate.requires_grad))
-        if needs_grad:
-            return _VSATiled.apply(q, k, v, gate, rows, vbs, vbs, topk, nb, be, scale,
-                                   token_major)
-        return _forward(q, k, v, gate, rows, vbs, vbs, topk, nb, be, scale, False,
-                        token_major)[0]
+        return launch.run(_spec(q, gate, topk, nb, be, 1.0 / math.sqrt(d), token_major), q, k, v,
+                      gate, None, vbs, vbs, rows)
