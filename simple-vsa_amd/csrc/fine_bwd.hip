@@ -918,10 +918,14 @@ __global__ __launch_bounds__((DkvCfg<D, BE>::NT)) __attribute__((amdgpu_waves_pe
   for (int round = 0;; ++round) {
     int j;
     if (ctr) {
-      if (threadIdx.x == 0) s_next = take_entry(ctr, xcd, per, from, last);  // the order entry
-      __syncthreads();
-      j = s_next;
-      if (j < 0) break;
+      j = 8 * (int)(blockIdx.x >> 3) + xcd;
+      if (round > 0) {
+        // the order entry
+        if (threadIdx.x == 0) s_next = take_entry(ctr, xcd, per, stride, from, last);
+        __syncthreads();
+        j = s_next;
+        if (j < 0) break;
+      }
       // an entry of its own index-order range lets the workgroup steal later
       if (threadIdx.x == 0 && from == 0 && !(tile_order[j] & kLongestFirst)) last = 8;
     } else {
@@ -1236,9 +1240,12 @@ sparse_dq_pp_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
   for (int round = 0;; ++round) {
     int tile;
     if (ctr) {  // as in sparse_fwd_pp_kernel
-      if (threadIdx.x == 0) s_next = take_entry(ctr, xcd, per, from, 8);
-      __syncthreads();
-      const int e = s_next;
+      int e = 8 * (int)(blockIdx.x >> 3) + xcd;
+      if (round > 0) {
+        if (threadIdx.x == 0) s_next = take_entry(ctr, xcd, per, stride, from, 8);
+        __syncthreads();
+        e = s_next;
+      }
       if (e < 0) break;
       tile = (e & 7) * per + (e >> 3);
     } else {

@@ -718,9 +718,9 @@ __device__ __forceinline__ void fwd_pp_tile(
 
 // Persistent: as many workgroups as the CUs hold (one each).  Workgroup i runs
 // on XCD i % 8 and takes the query blocks of that XCD's contiguous range (the
-// xcd_tile order), so one head's K/V stay in one XCD's L2: with scheduling
-// counters (sched_counters) the next block of the range, then the blocks left
-// in the other XCDs' ranges (take_entry; every block has the same topk chunks,
+// xcd_tile order), so one head's K/V stay in one XCD's L2: block i / 8 first,
+// then with scheduling counters (sched_counters) the next of the range, then
+// the blocks left in the other XCDs' ranges (take_entry; every block has the same topk chunks,
 // but the XCDs do not run equally fast: 0.6 % less time at c3 and 4.5 % at c4,
 // where 56.25 blocks per workgroup also left a fixed stride uneven); without,
 // a fixed stride over the range.
@@ -741,9 +741,12 @@ sparse_fwd_pp_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* 
   for (int round = 0;; ++round) {
     int tile;
     if (ctr) {
-      if (threadIdx.x == 0) s_next = take_entry(ctr, xcd, per, from, 8);
-      __syncthreads();
-      const int e = s_next;
+      int e = 8 * (int)(blockIdx.x >> 3) + xcd;
+      if (round > 0) {
+        if (threadIdx.x == 0) s_next = take_entry(ctr, xcd, per, stride, from, 8);
+        __syncthreads();
+        e = s_next;
+      }
       if (e < 0) break;
       tile = (e & 7) * per + (e >> 3);
     } else {
