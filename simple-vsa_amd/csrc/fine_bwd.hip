@@ -103,7 +103,7 @@ __device__ __forceinline__ void dq_epilogue(const f32x16 (&dqacc)[D / 32], int64
   }
 }
 
-template <typename T, int D, int BE, bool RASTER>
+template <typename T, int D, int BE, bool RASTER, bool SKIP>
 __global__ __launch_bounds__((DqCfg<D, BE>::NT)) __attribute__((amdgpu_waves_per_eu(DqCfg<D, BE>::WPE))) void
 sparse_dq_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                  const T* __restrict__ dout, const float* __restrict__ lse,
@@ -111,7 +111,8 @@ sparse_dq_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __re
                  const int32_t* __restrict__ kv_vbs, T* __restrict__ dq,
                  const T* __restrict__ dqc, const int32_t* __restrict__ q_vbs, int num_tiles,
                  int tiles_per_head, int sq, int skv, int qb, int kb, int topk, float c2,
-                 uint32_t qsign, float scale, const int32_t* __restrict__ orows, int64_t s_out, int heads) {
+                 uint32_t qsign, float scale, const int32_t* __restrict__ orows, int64_t s_out, int heads,
+                 int q_rows) {
   using C = DqCfg<D, BE>;
   using E = Elem<T>;
   typedef typename E::vec8 V8;
@@ -126,6 +127,8 @@ sparse_dq_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __re
   const int r = lane & 31, h = lane >> 5;
   const int myq = q0 + wave * 32 + r;
   const int64_t tok = (int64_t)b * sq + myq;
+  static_assert(!SKIP || C::QT == BE, "a workgroup holds a query block's first row");
+  const bool active = !SKIP || __builtin_amdgcn_readfirstlane(wave) * 32 < q_rows;
 
   V8 qf[D / 16], df[D / 16];
   {
@@ -221,6 +224,7 @@ sparse_dq_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __re
     const bool have2 = route.next(s2, ch2, kv2, nvb2);
     if (have2) dma(kv2, ch2, stage ^ 1);
 
+    if (active) {
     f32x16 sacc[C::NSM], pacc[C::NSM];
 #pragma unroll
     for (int smt = 0; smt < C::NSM; ++smt) sacc[smt] = pacc[smt] = f32x16{};
@@ -257,6 +261,7 @@ sparse_dq_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __re
 #pragma unroll
       for (int mt = 0; mt < D / 32; ++mt)
         dqacc[mt] = E::mfma32(k_tr(stage, mt, kk), bop, dqacc[mt]);
+    }
     }
     dma_wait();
     __syncthreads();
@@ -308,7 +313,7 @@ __device__ __forceinline__ void dkdv_tile(
     T* __restrict__ dk, T* __restrict__ dv, const T* __restrict__ dkc,
     const T* __restrict__ dvc, int tiles_per_head, int sq, int skv, int qb,
     int kb, int topk, float c2, uint32_t ksign, float scale,
-    const int32_t* __restrict__ orows, int64_t s_out, int heads) {
+    const int32_t* __restrict__ orows, int64_t s_out, int heads, int q_subs) {
   using C = DkvCfg<D, BE>;
   using E = Elem<T>;
   typedef typename E::vec8 V8;
@@ -352,7 +357,14 @@ __device__ __forceinline__ void dkdv_tile(
   const int64_t meta = (int64_t)b * kb + kvblk;
   const int nedge = counts[meta];
   const int32_t* seg = inverse + (int64_t)b * qb * topk + offsets[meta];
-  const int items = nedge * C::SUBS;
+  // An in-edge's items are the 32-row sub-tiles of its query block; at block
+  // 64 only the first one if no row of the second exists (q_subs 1).  At the
+  // larger blocks a count that is not the constant SUBS splits the four-step
+  // round's one CSR entry into four and spills (8 to 45 registers).  Forward +
+  // backward at 27-token blocks, 10 heads x 300 blocks: 3745 -> 2736 us at head
+  // dim 160, where this alone counts.
+  const int subs = BE == 64 && q_subs == 1 ? 1 : C::SUBS;
+  const int items = nedge * subs;
   // The pooled-gradient rows are one per key block: their dims are divided by
   // the count and rounded to T here, once per workgroup and dim, into LDS (in
   // the epilogue every lane would repeat them for its own key: about half of
@@ -428,21 +440,24 @@ __device__ __forceinline__ void dkdv_tile(
 
   // CSR segment staged in LDS, SEGMAX entries at a time (a scalar load per
   // item would put scalar-memory latency in front of every copy, a vector
-  // load would need vmcnt(0) and drain the ring).  The refill runs where every
-  // wave has finished with the previous entries (all waves call qblock_of at
-  // the same program point, between two barriers).  Entries [0, NT) were
-  // staged before the ring started.
+  // load would need vmcnt(0) and drain the ring).  A refill runs where every
+  // wave has finished with the previous entries (all waves are at the same
+  // program point), between two barriers: for each copy, or at block 64, where
+  // the edge of a copy is not known at compile time, once per round of the step
+  // loop for the NS items that the round copies (at block 128 and 256 that took
+  // 3 % longer: dK/dV 7.66 -> 7.93 ms at 40 heads x 40 960 tokens, head dim
+  // 128).  Entries [0, NT) were staged before the ring started.
+  constexpr bool REFILL_PER_ROUND = BE == 64 && D <= 128;
   int seg_lo = 0, seg_hi = C::NT;
-  auto qblock_of = [&](int item) {
-    const int e = item / C::SUBS;
-    if (e >= seg_hi) {
+  auto edge_of = [&](int item) { return BE == 64 ? item >> (subs - 1) : item / C::SUBS; };
+  auto stage_edges = [&](int first, int last) {  // items first .. last, those that exist
+    if (edge_of(min(last, items - 1)) >= seg_hi) {
       __syncthreads();
-      seg_lo = e;
-      seg_hi = e + C::SEGMAX;
+      seg_lo = edge_of(min(first, items - 1));
+      seg_hi = seg_lo + C::SEGMAX;
       for (int i = tid; i < C::SEGMAX && seg_lo + i < nedge; i += C::NT) sseg[i] = seg[seg_lo + i];
       __syncthreads();
     }
-    return __builtin_amdgcn_readfirstlane(sseg[e - seg_lo]);
   };
   struct Copy {
     const char* qsrc;
@@ -451,7 +466,10 @@ __device__ __forceinline__ void dkdv_tile(
   };
   auto copy_of = [&](int item) {
     Copy cp;
-    const int qrow0 = qblock_of(item) * BE + (item % C::SUBS) * C::QS;
+    if constexpr (!REFILL_PER_ROUND) stage_edges(item, item);
+    const int e = edge_of(item);
+    const int sub = BE == 64 ? item & (subs - 1) : item % C::SUBS;
+    const int qrow0 = __builtin_amdgcn_readfirstlane(sseg[e - seg_lo] * BE + sub * C::QS);
     cp.qsrc = reinterpret_cast<const char*>(qbase + (int64_t)qrow0 * D);
     cp.dsrc = reinterpret_cast<const char*>(dbase + (int64_t)qrow0 * D);
     cp.ssrc = lane < C::QS ? lbase + qrow0 + lane : ebase + qrow0 + (lane - C::QS);
@@ -602,6 +620,7 @@ __device__ __forceinline__ void dkdv_tile(
       static_assert(NS == 4, "the step sequence below is unrolled for NS = 4");
       int it = 0;
       for (; it + 4 <= items; it += 4) {
+        if constexpr (REFILL_PER_ROUND) stage_edges(it + NS, it + 2 * NS - 1);
         sstep(I0{}, it);
         sstep(I1{}, it + 1);
         sstep(I2{}, it + 2);
@@ -775,10 +794,8 @@ __device__ __forceinline__ void dkdv_tile(
 #pragma unroll
       for (int x = NA + NC + L; x < NA + NC + 4; ++x) issue(x);
       // descriptor of the copy issued by the next step (its CSR entry is an
-      // LDS read, kept off the next step's critical path).  It comes after
-      // both MFMA phases: the CSR refill branch inside it splits the code, and
-      // placed between the phases it let the compiler sink B(i) (used only by
-      // C(i)) past the branch, out from under the MFMAs of A(i+1).
+      // LDS read, kept off the next step's critical path), after both MFMA
+      // phases: a refill branch inside it would split the code between them.
       const int nn = it + NS;
       cpn = copy_of(nn < items ? nn : items - 1);
     };
@@ -789,6 +806,7 @@ __device__ __forceinline__ void dkdv_tile(
     static_assert(NS == 4, "the step sequence below is unrolled for NS = 4");
     int it = 0;
     for (; it + 4 <= items; it += 4) {
+      if constexpr (REFILL_PER_ROUND) stage_edges(it + NS, it + 2 * NS - 1);
       step(I0{}, it, sA, pA, sB, pB, lA, dA, lB, dB, preA, preB);
       step(I1{}, it + 1, sB, pB, sA, pA, lB, dB, lA, dA, preB, preA);
       step(I2{}, it + 2, sA, pA, sB, pB, lA, dA, lB, dB, preA, preB);
@@ -894,7 +912,7 @@ __global__ __launch_bounds__((DkvCfg<D, BE>::NT)) __attribute__((amdgpu_waves_pe
     T* __restrict__ dk, T* __restrict__ dv, const T* __restrict__ dkc,
     const T* __restrict__ dvc, int num_tiles, int tiles_per_head, int sq, int skv, int qb,
     int kb, int topk, float c2, uint32_t ksign, float scale, int32_t* __restrict__ tile_order,
-    const int32_t* __restrict__ orows, int64_t s_out, int heads) {
+    const int32_t* __restrict__ orows, int64_t s_out, int heads, int q_subs) {
   __shared__ DkvShared<T, D, BE> sh;
   if constexpr (DkvCfg<D, BE>::NSPLIT > 1) {
     // head_dim 256: one tile per workgroup (the loop's state would push the
@@ -904,7 +922,7 @@ __global__ __launch_bounds__((DkvCfg<D, BE>::NT)) __attribute__((amdgpu_waves_pe
     if (tile_s < num_tiles)
       dkdv_tile<T, D, BE, RASTER>(sh, tile_s, q, k, v, dout, lse, delta, counts, offsets,
                                   inverse, kv_vbs, dk, dv, dkc, dvc, tiles_per_head, sq, skv, qb,
-                                  kb, topk, c2, ksign, scale, orows, s_out, heads);
+                                  kb, topk, c2, ksign, scale, orows, s_out, heads, q_subs);
     return;
   }
   __shared__ int s_next;
@@ -937,7 +955,7 @@ __global__ __launch_bounds__((DkvCfg<D, BE>::NT)) __attribute__((amdgpu_waves_pe
     if (tile_s < num_tiles)
       dkdv_tile<T, D, BE, RASTER>(sh, tile_s, q, k, v, dout, lse, delta, counts, offsets,
                                   inverse, kv_vbs, dk, dv, dkc, dvc, tiles_per_head, sq, skv, qb,
-                                  kb, topk, c2, ksign, scale, orows, s_out, heads);
+                                  kb, topk, c2, ksign, scale, orows, s_out, heads, q_subs);
     dma_wait();       // this wave's trailing copies land before the LDS is reused
     __syncthreads();  // and every wave is done with it (and with s_next)
   }
@@ -1289,18 +1307,21 @@ template <typename T, int D, int BE, bool RASTER = false>
 static int launch_dq(const void* q, const void* k, const void* v, const void* dout,
                      const float* lse, const float* delta, const int32_t* selected,
                      const int32_t* kv_vbs, void* dq, const void* dqc, const int32_t* q_vbs,
-                     int64_t bh, int64_t sq, int64_t skv, int topk, float scale,
+                     int64_t bh, int64_t sq, int64_t skv, int topk, float scale, int rows,
                      hipStream_t stream, const int32_t* orows = nullptr, int64_t s_out = 0, int heads = 0) {
   using C = DqCfg<D, BE>;
   const int tph = (int)(sq / C::QT);
   const int64_t tiles = bh * tph;
   if (tiles > (1LL << 30)) return VSA_ERR_SHAPE;
   const int grid = (int)(((tiles + 7) / 8) * 8);
-  hipLaunchKernelGGL((sparse_dq_kernel<T, D, BE, RASTER>), dim3(grid), dim3(C::NT), 0, stream,
+  auto* kernel = sparse_dq_kernel<T, D, BE, RASTER, false>;
+  if constexpr (!RASTER && BE < 256 && D <= 128)  // as in launch_fwd
+    if (rows <= BE - 32) kernel = sparse_dq_kernel<T, D, BE, RASTER, true>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(C::NT), 0, stream,
                      (const T*)q, (const T*)k, (const T*)v, (const T*)dout, lse, delta, selected,
                      kv_vbs, (T*)dq, (const T*)dqc, q_vbs, (int)tiles, tph, (int)sq, (int)skv,
                      (int)(sq / BE), (int)(skv / BE), topk, fabsf(scale) * kLog2e,
-                     scale < 0.f ? 0x80008000u : 0u, scale, orows, s_out, heads);
+                     scale < 0.f ? 0x80008000u : 0u, scale, orows, s_out, heads, rows);
   return vsa_check_launch();
 }
 
@@ -1309,7 +1330,7 @@ static int launch_dkdv(const void* q, const void* k, const void* v, const void* 
                        const float* lse, const float* delta, const int32_t* counts,
                        const int32_t* offsets, const int32_t* inverse, const int32_t* kv_vbs,
                        void* dk, void* dv, const void* dkc, const void* dvc, int64_t bh,
-                       int64_t sq, int64_t skv, int topk, float scale, int32_t* tile_order,
+                       int64_t sq, int64_t skv, int topk, float scale, int rows, int32_t* tile_order,
                        hipStream_t stream, const int32_t* orows = nullptr, int64_t s_out = 0, int heads = 0) {
   using C = DkvCfg<D, BE>;
   const int tph = (int)(skv / C::KT);
@@ -1325,7 +1346,7 @@ static int launch_dkdv(const void* q, const void* k, const void* v, const void* 
                      offsets, inverse, kv_vbs, (T*)dk, (T*)dv, (const T*)dkc, (const T*)dvc,
                      (int)tiles, tph, (int)sq, (int)skv, (int)(sq / BE), (int)(skv / BE), topk,
                      fabsf(scale) * kLog2e, scale < 0.f ? 0x80008000u : 0u, scale, tile_order,
-                     orows, s_out, heads);
+                     orows, s_out, heads, (rows + C::QS - 1) / C::QS);
   return vsa_check_launch();
 }
 
@@ -1494,12 +1515,12 @@ using namespace vsa;
 #define VSA_BWD_SHAPES(X) \
   X(128, 256) X(128, 128) X(128, 64) X(64, 256) X(64, 128) X(64, 64) X(256, 256) X(256, 128) X(256, 64)
 
-extern "C" int vsa_sparse_bwd_dq(const void* q, const void* k, const void* v, const void* dout,
-                                 const float* lse, const float* delta, const int32_t* selected,
-                                 const int32_t* kv_vbs, void* dq, const void* d_q_c,
-                                 const int32_t* q_vbs, int64_t bh, int64_t sq, int64_t skv,
-                                 int32_t D, int32_t be, int32_t topk, float scale, int32_t dtype,
-                                 void* stream) {
+int vsa::sparse_bwd_dq_rows(int rows, const void* q, const void* k, const void* v,
+                            const void* dout, const float* lse, const float* delta,
+                            const int32_t* selected, const int32_t* kv_vbs, void* dq,
+                            const void* d_q_c, const int32_t* q_vbs, int64_t bh, int64_t sq,
+                            int64_t skv, int32_t D, int32_t be, int32_t topk, float scale,
+                            int32_t dtype, void* stream) {
   if (!q || !k || !v || !dout || !lse || !delta || !selected || !kv_vbs || !dq) return VSA_ERR_NULL;
   if (d_q_c && !q_vbs) return VSA_ERR_NULL;
   if (!vsa_aligned<16>(q, k, v, dout, dq, d_q_c) || !vsa_aligned<4>(lse, delta, selected, kv_vbs, q_vbs))
@@ -1528,10 +1549,20 @@ extern "C" int vsa_sparse_bwd_dq(const void* q, const void* k, const void* v, co
 #define VSA_DQ_CASE(DD, BB)                                                                  \
   if (D == DD && be == BB)                                                                   \
     return launch_dq<T, DD, BB>(q, k, v, dout, lse, delta, selected, kv_vbs, dq, d_q_c, q_vbs, \
-                                bh, sq, skv, topk, scale, s);
+                                bh, sq, skv, topk, scale, rows, s);
   VSA_DISPATCH_MFMA(dtype, T, { VSA_BWD_SHAPES(VSA_DQ_CASE) });
 #undef VSA_DQ_CASE
   return VSA_ERR_UNSUPPORTED;
+}
+
+extern "C" int vsa_sparse_bwd_dq(const void* q, const void* k, const void* v, const void* dout,
+                                 const float* lse, const float* delta, const int32_t* selected,
+                                 const int32_t* kv_vbs, void* dq, const void* d_q_c,
+                                 const int32_t* q_vbs, int64_t bh, int64_t sq, int64_t skv,
+                                 int32_t D, int32_t be, int32_t topk, float scale, int32_t dtype,
+                                 void* stream) {
+  return sparse_bwd_dq_rows(be, q, k, v, dout, lse, delta, selected, kv_vbs, dq,
+                            d_q_c, q_vbs, bh, sq, skv, D, be, topk, scale, dtype, stream);
 }
 
 extern "C" int vsa_dkdv_tile_order(const int32_t* counts, int32_t* tile_order,
@@ -1551,14 +1582,13 @@ extern "C" int vsa_dkdv_tile_order(const int32_t* counts, int32_t* tile_order,
   return vsa_check_launch();
 }
 
-extern "C" int vsa_sparse_bwd_dkdv(const void* q, const void* k, const void* v,
-                                   const void* dout, const float* lse, const float* delta,
-                                   const int32_t* counts, const int32_t* offsets,
-                                   const int32_t* inverse, const int32_t* kv_vbs, void* dk,
-                                   void* dv, const void* d_k_c, const void* d_v_c, int64_t bh,
-                                   int64_t sq, int64_t skv, int32_t D, int32_t be, int32_t topk,
-                                   float scale, int32_t* tile_order, int32_t dtype,
-                                   void* stream) {
+int vsa::sparse_bwd_dkdv_rows(int rows, const void* q, const void* k, const void* v,
+                              const void* dout, const float* lse, const float* delta,
+                              const int32_t* counts, const int32_t* offsets,
+                              const int32_t* inverse, const int32_t* kv_vbs, void* dk, void* dv,
+                              const void* d_k_c, const void* d_v_c, int64_t bh, int64_t sq,
+                              int64_t skv, int32_t D, int32_t be, int32_t topk, float scale,
+                              int32_t* tile_order, int32_t dtype, void* stream) {
   if (!q || !k || !v || !dout || !lse || !delta || !counts || !offsets || !inverse || !kv_vbs ||
       !dk || !dv)
     return VSA_ERR_NULL;
@@ -1576,11 +1606,23 @@ extern "C" int vsa_sparse_bwd_dkdv(const void* q, const void* k, const void* v,
 #define VSA_DKDV_CASE(DD, BB)                                                                \
   if (D == DD && be == BB)                                                                   \
     return launch_dkdv<T, DD, BB>(q, k, v, dout, lse, delta, counts, offsets, inverse,       \
-                                  kv_vbs, dk, dv, d_k_c, d_v_c, bh, sq, skv, topk, scale, \
+                                  kv_vbs, dk, dv, d_k_c, d_v_c, bh, sq, skv, topk, scale, rows, \
                                   tile_order, s);
   VSA_DISPATCH_MFMA(dtype, T, { VSA_BWD_SHAPES(VSA_DKDV_CASE) });
 #undef VSA_DKDV_CASE
   return VSA_ERR_UNSUPPORTED;
+}
+
+extern "C" int vsa_sparse_bwd_dkdv(const void* q, const void* k, const void* v, const void* dout,
+                                   const float* lse, const float* delta, const int32_t* counts,
+                                   const int32_t* offsets, const int32_t* inverse,
+                                   const int32_t* kv_vbs, void* dk, void* dv, const void* d_k_c,
+                                   const void* d_v_c, int64_t bh, int64_t sq, int64_t skv,
+                                   int32_t D, int32_t be, int32_t topk, float scale,
+                                   int32_t* tile_order, int32_t dtype, void* stream) {
+  return sparse_bwd_dkdv_rows(be, q, k, v, dout, lse, delta, counts, offsets,
+                              inverse, kv_vbs, dk, dv, d_k_c, d_v_c, bh, sq, skv, D, be, topk,
+                              scale, tile_order, dtype, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1697,7 +1739,8 @@ extern "C" int vsa_sparse_bwd_dq_tiled(const void* q, const void* k, const void*
       return launch_dq_pp<T, DD, true>(q, k, v, dout, lse, delta, selected, kv_vbs, dq, d_q_c, \
                                        q_vbs, bh, sq, skv, topk, scale, s, slot_rows, s_out, heads); \
     return launch_dq<T, DD, BB, true>(q, k, v, dout, lse, delta, selected, kv_vbs, dq, d_q_c, \
-                                      q_vbs, bh, sq, skv, topk, scale, s, slot_rows, s_out, heads);  \
+                                      q_vbs, bh, sq, skv, topk, scale, be, s, slot_rows, s_out,    \
+                                      heads);                                                    \
   }
   VSA_DISPATCH_MFMA(dtype, T, { VSA_TILED_SHAPES(VSA_DQ_TILED_CASE) });
 #undef VSA_DQ_TILED_CASE
@@ -1730,7 +1773,7 @@ extern "C" int vsa_sparse_bwd_dkdv_tiled(const void* q, const void* k, const voi
   if (D == DD && be == BB)                                                                   \
     return launch_dkdv<T, DD, BB, true>(q, k, v, dout, lse, delta, counts, offsets, inverse, \
                                         kv_vbs, dk, dv, d_k_c, d_v_c, bh, sq, skv, topk,     \
-                                        scale, tile_order, s, slot_rows, s_out, heads);
+                                        scale, be, tile_order, s, slot_rows, s_out, heads);
   VSA_DISPATCH_MFMA(dtype, T, { VSA_TILED_SHAPES(VSA_DKDV_TILED_CASE) });
 #undef VSA_DKDV_TILED_CASE
   return VSA_ERR_UNSUPPORTED;

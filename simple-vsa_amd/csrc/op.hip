@@ -248,9 +248,9 @@ extern "C" int vsa_op_fwd(const vsa_op* op, void* out, void* saved, void* scratc
     return vsa_sparse_fwd_tiled(q, kk, v, sel, op->kv_vbs, res, k.fine, k.lse, k.outc, gate,
                                 op->gate_mode, op->slot_rows, op->s_out, op->heads, op->bh, d.sq,
                                 d.skv, d.D, d.be, op->topk, op->scale, op->dtype, stream);
-  VSA_TRY(vsa_sparse_fwd(q, kk, v, sel, op->kv_vbs, res, d.full ? k.fine : nullptr, k.lse, k.outc,
-                         gate, d.full ? op->gate_mode : 0, op->gate_heads, op->bh, d.sq, d.skv,
-                         d.D, d.be, op->topk, op->scale, op->dtype, stream));
+  VSA_TRY(sparse_fwd_rows(op->block, q, kk, v, sel, op->kv_vbs, res, d.full ? k.fine : nullptr,
+                          k.lse, k.outc, gate, d.full ? op->gate_mode : 0, op->gate_heads, op->bh,
+                          d.sq, d.skv, d.D, d.be, op->topk, op->scale, op->dtype, stream));
   if (d.padded) {
     Moves mv(op, d, false);
     mv.rows(res, out, d.qb);
@@ -318,10 +318,10 @@ extern "C" int vsa_op_bwd(const vsa_op* op, const void* out, const void* dout, v
                                      op->heads, op->bh, d.sq, d.skv, d.D, d.be, op->topk,
                                      op->scale, b.order, op->dtype, stream);
   }
-  VSA_TRY(vsa_sparse_bwd_dq(q, kk, v, g, k.lse, b.delta, sel, op->kv_vbs, gq, b.dqc,
+  VSA_TRY(sparse_bwd_dq_rows(op->block, q, kk, v, g, k.lse, b.delta, sel, op->kv_vbs, gq, b.dqc,
                             d.full ? op->q_vbs : nullptr, op->bh, d.sq, d.skv, d.D, d.be,
                             op->topk, op->scale, op->dtype, stream));
-  VSA_TRY(vsa_sparse_bwd_dkdv(q, kk, v, g, k.lse, b.delta, b.counts, b.offsets, b.inverse,
+  VSA_TRY(sparse_bwd_dkdv_rows(op->block, q, kk, v, g, k.lse, b.delta, b.counts, b.offsets, b.inverse,
                               op->kv_vbs, gk, gv, b.dkc, b.dvc, op->bh, d.sq, d.skv, d.D, d.be,
                               op->topk, op->scale, b.order, op->dtype, stream));
   if (d.padded) {

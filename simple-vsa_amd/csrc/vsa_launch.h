@@ -85,6 +85,28 @@ struct BlockMove {
   int n, be, kbe;
 };
 int block_move(BlockMove& m, bool pad, hipStream_t s);
+// vsa_sparse_fwd / _bwd_dq / _bwd_dkdv for query blocks of which only the first
+// `rows` rows exist (the caller's volume, where the blocks are padded to a
+// volume the kernels have); the others are zero in q and dout, and no one reads
+// their results.  The bf16 / fp16 forward and dQ multiply nothing for 32 rows
+// that do not exist (their results are those of rows of zeros), and dK / dV at
+// block 64 takes no items of them.
+int sparse_fwd_rows(int rows, const void* q, const void* k, const void* v, const int32_t* selected,
+                    const int32_t* kv_vbs, void* out, void* fine_out, float* lse,
+                    const void* out_c, const void* gate, int32_t gate_mode, int32_t gate_heads,
+                    int64_t bh, int64_t sq, int64_t skv, int32_t D, int32_t be, int32_t topk,
+                    float scale, int32_t dtype, void* stream);
+int sparse_bwd_dq_rows(int rows, const void* q, const void* k, const void* v, const void* dout,
+                       const float* lse, const float* delta, const int32_t* selected,
+                       const int32_t* kv_vbs, void* dq, const void* d_q_c, const int32_t* q_vbs,
+                       int64_t bh, int64_t sq, int64_t skv, int32_t D, int32_t be, int32_t topk,
+                       float scale, int32_t dtype, void* stream);
+int sparse_bwd_dkdv_rows(int rows, const void* q, const void* k, const void* v, const void* dout,
+                         const float* lse, const float* delta, const int32_t* counts,
+                         const int32_t* offsets, const int32_t* inverse, const int32_t* kv_vbs,
+                         void* dk, void* dv, const void* d_k_c, const void* d_v_c, int64_t bh,
+                         int64_t sq, int64_t skv, int32_t D, int32_t be, int32_t topk, float scale,
+                         int32_t* tile_order, int32_t dtype, void* stream);
 // Scheduling counters (take_entry) of the persistent forward and dQ kernels for
 // launches on stream s, from a file-scope device array (common.hip): one slot
 // of zeroed counters per (device, stream), which every launch leaves zeroed.
