@@ -24,9 +24,9 @@ rounding below fp32 anywhere on its path).  Other shapes the reference accepts
 on the GPU (volume in [1, 128], head_dim <= 256; triton_impl.py:379-384) run on
 the same kernels after zero-padding each block to the next kernel volume and
 the head dim to the next kernel width; the softmax scale stays 1/sqrt(head_dim)
-of the caller's tensors.  Padded query rows are computed and dropped, padded
-keys are masked by the block sizes, padded channels are zero in every dot
-product.
+of the caller's tensors.  Padded query rows are dropped (and 32 of them together
+are not multiplied), padded keys are masked by the block sizes, padded channels
+are zero in every dot product.
 
 Both ops run a whole pass as one call into the library (``launch``); the
 functions here check, convert and pick the op's sizes.
