@@ -122,6 +122,8 @@ class Op(torch.autograd.Function):
         dout = dout.contiguous()
         if dout.data_ptr() % 16:
             dout = dout.clone()
+        if saved.data_ptr() % 256:  # what a saved-tensor hook gave back
+            saved = saved.clone()
         dev = dout.device
         dq = torch.empty(q_shape, dtype=dout.dtype, device=dev)
         dk = torch.empty(k_shape, dtype=dout.dtype, device=dev)

@@ -95,3 +95,23 @@ def test_route_op_equals_its_steps(be, d, dt):
     delta, _, _ = M.backward_prep(o, dp, kbe)
     grads = M.sparse_backward(qp, kp, vp, dp, lse, delta, sel, vbs, kbe, 0.2)
     _same(got, [unpad(x) for x in (o, *grads)], ["out", "dq", "dk", "dv"])
+
+
+def test_saved_tensors_come_back_unaligned():
+    """A saved-tensor hook may give the kept workspace back at any address."""
+    from vsa_mi355x import mi355x as M
+    q, k, v, do = (x.requires_grad_() for x in _rand(3, [(1, 2, 320, 64)] * 4, BF))
+    vbs = torch.full((5,), 64, dtype=torch.int32, device=DEV)
+
+    def unpack(t):
+        if t.dtype != torch.uint8:
+            return t
+        return torch.empty(t.numel() + 16, dtype=torch.uint8, device=DEV)[16:].copy_(t)
+
+    def grads():
+        return torch.autograd.grad(M.mi355x_vsa(q, k, v, vbs, vbs, 2, (4, 4, 4)), [q, k, v],
+                                   do.detach())
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        got = grads()
+    _same(got, grads(), ["dq", "dk", "dv"])
