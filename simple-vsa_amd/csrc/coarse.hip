@@ -625,12 +625,14 @@ __global__ __launch_bounds__(kNT) void coarse_bwd_cols_mfma_kernel(
   for (int t = wave; t < ntile; t += kWaves) {
     // B operand: the weights [q][key r] of the 16 queries this lane feeds (rows
     // past the end are clamped, loaded and zeroed: a load under the condition
-    // would be a branch and a wait per value)
+    // would be a branch and a wait per value).  The tile's first row is a 64-bit
+    // offset (any number of query blocks is taken), the 32 rows in it 32-bit ones.
     float w[16];
     RowStage<T, D, DH> st;
+    const float* wt = weights + (int64_t)t * 32 * kb + mykey;
+    const int last = qb - 1 - t * 32;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)  // offsets < 2^28: at most 16 000 blocks each way
-      w[i] = weights[(uint32_t)min(t * 32 + acc_row(i, h), qb - 1) * kb + mykey];
+    for (int i = 0; i < 16; ++i) w[i] = wt[min(acc_row(i, h), last) * kb];
     st.load(rows, t * 32, qb);
 #pragma unroll
     for (int i = 0; i < 16; ++i)

@@ -42,6 +42,31 @@ def test_coarse_against_the_oracle(D, qb, kb):
         assert rel <= 1e-2, (what, rel)
 
 
+def test_columns_past_2_32_weights():
+    """d_k_c and d_v_c of a head with more than 2^32 probabilities (16 000 key
+    blocks; the last query rows lie past them): rows without weight add exact
+    zeros and each key has one row with weight, so the rows that have some give
+    the same by themselves, bit for bit."""
+    from vsa_mi355x import mi355x as M
+    kb, D = 16000, 64
+    qb = (1 << 32) // kb + 100
+    if torch.cuda.mem_get_info()[0] < 48 << 30:
+        pytest.skip("needs 35 GB of free HBM")
+    g = torch.Generator(device=DEV).manual_seed(1)
+    qc, kc, vc, do = (torch.randn(1, 1, n, D, generator=g, device=DEV).bfloat16()
+                      for n in (qb, kb, kb, qb))
+    rows = torch.cat([torch.arange(40), torch.arange(qb - 150, qb)]).to(DEV)
+    keys = torch.arange(rows.numel(), device=DEV) * 2
+    probs = torch.zeros(1, 1, qb, kb, device=DEV)
+    probs[0, 0, rows, keys] = 0.25
+    probs[0, 0, rows, keys + 1] = 0.75
+    got = M.coarse_backward(qc, kc, vc, probs, do, 0.125)
+    ref = M.coarse_backward(qc[:, :, rows], kc, vc, probs[:, :, rows], do[:, :, rows], 0.125)
+    assert all((x != 0).any() for x in ref)
+    assert torch.equal(got[0][:, :, rows], ref[0])
+    assert torch.equal(got[1], ref[1]) and torch.equal(got[2], ref[2])
+
+
 @pytest.mark.parametrize("kb", [63, 64, 65, 128, 129, 512, 513, 1024, 1025, 2048, 2049])
 @pytest.mark.parametrize("kind", ["bf16", "fp32", "low_bits", "few"])
 def test_topk_against_the_rule(kb, kind):
