@@ -297,6 +297,21 @@ __device__ __forceinline__ Split8 split_acc(const f32x16& acc, int kk) {
   return split8(x);
 }
 
+// The same of a tile of any values (dS, where an infinite dO or V makes some).
+__device__ __forceinline__ void split_acc_any(const f32x16& acc, Split8 (&s)[2]) {
+  float x[2][8];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) x[e >> 3][e & 7] = acc[e];
+  const float mx = vmax(absmax8(x[0]), absmax8(x[1]));
+  if (__any(!(mx < INFINITY))) {
+    s[0] = split8_any(x[0]);
+    s[1] = split8_any(x[1]);
+  } else {
+    s[0] = split8(x[0]);
+    s[1] = split8(x[1]);
+  }
+}
+
 // Steps 0 .. N-1 of a product: step st's LDS operand `load(st)` is read one step
 // ahead of its use in `mul(st, operand)`.  The scheduler keeps to the steps (it
 // would otherwise read many operands ahead and spill).
@@ -605,7 +620,8 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
       const float p = key < nk ? exp2f(fmaf(sacc[i], c2, -my_lse)) : 0.f;
       sacc[i] = p * (pacc[i] - my_delta);
     }
-    const Split8 ds[2] = {split_acc(sacc, 0), split_acc(sacc, 1)};
+    Split8 ds[2];
+    split_acc_any(sacc, ds);
     pipelined<D / 16>(
         [&](int x) { return tile_col<D>(kt, 32 * (x % (D / 32)), x / (D / 32)); },
         [&](int x, const Split8& a) {
@@ -739,7 +755,8 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
         [&](int x, const Split8& a) {
           dva[x % (D / 32)] = mma6(a, p[x / (D / 32)], dva[x % (D / 32)]);
         });
-    const Split8 ds[2] = {split_acc(pacc, 0), split_acc(pacc, 1)};
+    Split8 ds[2];
+    split_acc_any(pacc, ds);
     pipelined<D / 16>(  // dK^T += Q^T dS
         [&](int x) { return tile_col<D>(qt, 32 * (x % (D / 32)), x / (D / 32)); },
         [&](int x, const Split8& a) {

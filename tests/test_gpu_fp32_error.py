@@ -1,0 +1,43 @@
+"""Errors of the fp32 kernels at head dims 64 / 128 (split bf16 products) that
+random data does not show."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+SHAPES = [(64, 64), (64, 128), (128, 64), (256, 64), (256, 128)]
+
+
+@pytest.fixture(autouse=True)
+def _gpu_only():
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+
+
+
+
+@pytest.mark.parametrize("be,D", SHAPES)
+def test_infinite_gradients_stay_infinite(be, D):
+    """One infinite value in dO makes its row of dS -inf at the keys whose v has
+    the other sign there: those keys' dK is infinite with the sign of -q, the
+    other keys' NaN."""
+    from vsa_mi355x import mi355x as M
+    nb = 3
+    g = torch.Generator(device=DEV).manual_seed(be + D)
+    q, k, v, do = (torch.randn(1, 1, be * nb, D, generator=g, device=DEV) for _ in range(4))
+    sel = torch.arange(nb, device=DEV, dtype=torch.int32).expand(1, 1, nb, nb).contiguous()
+    vbs = torch.full((nb,), be, dtype=torch.int32, device=DEV)
+    do[0, 0, 40, 3] = math.inf
+    leaves = [x.clone().requires_grad_() for x in (q, k, v)]
+    out = M.mi355x_sparse_attention(*leaves, sel, vbs, block_size=(1, 1, be))
+    got = torch.autograd.grad(out, leaves, do)[1][0, 0].double()
+    q, k, v, do = (x[0, 0].double().cpu() for x in (q, k, v, do))
+    p = torch.softmax(q @ k.T / math.sqrt(D), -1)
+    delta = ((p @ v) * do).sum(-1, keepdim=True)
+    ref = ((p * (do @ v.T - delta)).T @ q / math.sqrt(D)).to(DEV)
+    assert torch.isinf(ref).any() and torch.isnan(ref).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)])
