@@ -186,6 +186,18 @@ __device__ __forceinline__ f32x16 mma6(const Split8& a, const Split8& b, f32x16 
   return E::mfma32(a.hi, b.hi, acc);
 }
 
+// b . a in the order of mma6(b, a): the same sum bit for bit with the operands'
+// places exchanged.
+__device__ __forceinline__ f32x16 mma6_as_ba(const Split8& a, const Split8& b, f32x16 acc) {
+  using E = Elem<bf16_t>;
+  acc = E::mfma32(a.hi, b.lo, acc);
+  acc = E::mfma32(a.lo, b.hi, acc);
+  acc = E::mfma32(a.mid, b.mid, acc);
+  acc = E::mfma32(a.hi, b.mid, acc);
+  acc = E::mfma32(a.mid, b.hi, acc);
+  return E::mfma32(a.hi, b.hi, acc);
+}
+
 // This lane's row of an operand held in registers: dims 16 ks + 8h .. +7.
 template <int D>
 __device__ __forceinline__ void load_split(Split8 (&f)[D / 16], const float* __restrict__ row,
@@ -715,10 +727,12 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
     bf16_t* qnext = qs_ + (C::QBUF == 2 ? buf ^ 1 : 0) * SplitTile<D>::ELEMS;
     __syncthreads();  // Q and statistics written; every wave is done with dO
     f32x16 sacc = f32x16{}, pacc = f32x16{};
-    // S (queries x keys), lane column = key r
+    // S (queries x keys), lane column = key r, as the forward summed it: P is
+    // exp2 of its difference to a sum of the forward's S, which shares S's
+    // rounding only then
     pipelined<D / 16>([&](int ks) { return tile_row<D>(qt, r, ks, h); },
                       [&](int ks, const Split8& a) {
-                        sacc = mma6(a, kf[ks], sacc);
+                        sacc = mma6_as_ba(a, kf[ks], sacc);
                         const int i = Copy::piece_after(ks, D / 16, C::FIRST);
                         if (i >= 0) oc.put(i, os_);
                       });

@@ -17,6 +17,10 @@ def _gpu_only():
         pytest.skip("needs an MI355X")
 
 
+def _own_block(H, nb):
+    """Every query block routed to its own key block, of which one key is valid."""
+    sel = torch.arange(nb, device=DEV, dtype=torch.int32).view(1, 1, nb, 1)
+    return sel.expand(1, H, nb, 1).contiguous(), torch.ones(nb, dtype=torch.int32, device=DEV)
 
 
 @pytest.mark.parametrize("be,D", SHAPES)
@@ -41,3 +45,23 @@ def test_infinite_gradients_stay_infinite(be, D):
     assert torch.isinf(ref).any() and torch.isnan(ref).any()
     assert torch.equal(torch.isnan(got), torch.isnan(ref))
     assert torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)])
+
+
+@pytest.mark.parametrize("be,D", SHAPES)
+def test_weights_come_from_the_scores_of_the_forward(be, D):
+    """With one key a row and exponents of exactly the score (scale ln 2, whose
+    product with log2 e rounds to 1), P is exp2(S - S): 1 exactly if dK / dV sums
+    S as the forward does, so dV is what it is for scores of zero."""
+    from vsa_mi355x import mi355x as M
+    nb, H = 5, 3
+    g = torch.Generator(device=DEV).manual_seed(be + D)
+    q, k, v, do = (1 + torch.rand(1, H, be * nb, D, generator=g, device=DEV) for _ in range(4))
+    sel, vbs = _own_block(H, nb)
+
+    def dv(q):
+        leaves = [x.clone().requires_grad_() for x in (q, k, v)]
+        out = M.mi355x_sparse_attention(*leaves, sel, vbs, block_size=(1, 1, be),
+                                        sm_scale=0.6931471824645996)
+        return torch.autograd.grad(out, leaves, do)[2]
+
+    assert torch.equal(dv(q), dv(torch.zeros_like(q)))
