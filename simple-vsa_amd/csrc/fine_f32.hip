@@ -389,13 +389,22 @@ struct RouteCursor {
 // Forward: out = softmax(q k^T scale) v over the selected blocks, LSE base 2,
 // combine `out_c * gate` in the epilogue.  Per wave (32 queries) and 32-key
 // chunk: S^T = K Q^T, online softmax per lane-query (lane halves hold 16 keys
-// each, joined by a permlane swap), O^T += V^T P^T.  The exponents' offset is
-// kSplitSlack above a row's max when it moves, and moves only when a chunk
-// passes it: weights stay <= 1 and O is rescaled on few chunks.  The next V tile is split and written under
-// the S products, the next K tile under the O products: one buffer each and
-// two barriers a chunk.
+// each, joined by a permlane swap), O^T += V^T P^T.  A row's offset of the
+// exponents is a chunk's max and moves only when a later chunk's passes it by
+// more than kMaxSlack: O is rescaled on few chunks, and the exponents of the
+// largest weights stay near 0, where fp32 resolves them.  The weights are kept
+// as 2^-kMaxSlack of their value, at most 1, so that no product passes v's
+// largest.  The next V tile is split and written under the S products, the next
+// K tile under the O products: one buffer each and two barriers a chunk.
 // ---------------------------------------------------------------------------
-constexpr float kSplitSlack = 8.0f;
+constexpr int kMaxSlack = 4;
+
+// 2^(x - kMaxSlack), with the rounding of exp2f(x).
+__device__ __forceinline__ float weight_exp2(float x) {
+  const bool tiny = x < -126.0f;  // the instruction's results end at 2^-126
+  return __builtin_ldexpf(__builtin_amdgcn_exp2f(tiny ? x + 64.0f : x),
+                          tiny ? -64 - kMaxSlack : -kMaxSlack);
+}
 
 template <int D, int BE>
 __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
@@ -425,7 +434,7 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
   f32x16 o[D / 32];
 #pragma unroll
   for (int mt = 0; mt < D / 32; ++mt) o[mt] = f32x16{};
-  float m = -INFINITY, l = 0.f;  // offset of the exponents (log2 units), this half's partial sum
+  float m = -INFINITY, l = 0.f;  // offset of the exponents (log2 units), this half's sum of weights
   const float* kbase = k + b * (int64_t)skv * D;
   const float* vbase = v + b * (int64_t)skv * D;
   RouteCursor<BE> cur{selected + (b * qb + qblk) * topk, kv_vbs, topk, kb};
@@ -457,9 +466,9 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
     cmax = pair_max32(cmax);
     // a row moves its own offset only, so that its values never depend on the
     // other rows of the wave (a NaN moves it too, and stays)
-    const bool grow = !(cmax <= m);
+    const bool grow = !(cmax <= m + (float)kMaxSlack);
     if (__any(grow)) {
-      const float mnew = grow ? cmax + kSplitSlack : m;
+      const float mnew = grow ? cmax : m;
       const float alpha = exp2f(m - mnew);
       l *= alpha;
 #pragma unroll
@@ -469,7 +478,7 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      sacc[i] = exp2f(sacc[i] - m);
+      sacc[i] = weight_exp2(sacc[i] - m);
       psum += sacc[i];
     }
     l += psum;
@@ -490,7 +499,7 @@ __global__ __launch_bounds__((SplitCfg<D, BE>::NT))
   // epilogue: normalise, fused combine, LSE
   const float ltot = pair_sum32(l);
   const float inv = 1.0f / ltot;
-  if (lse != nullptr && h == 0) lse[tok] = m + log2f(ltot);
+  if (lse != nullptr && h == 0) lse[tok] = m + log2f(__builtin_ldexpf(ltot, kMaxSlack));
   const float* ocrow = outc ? outc + (b * qb + qblk) * D : nullptr;
   const float* grow = nullptr;
   float gtok = 1.f;

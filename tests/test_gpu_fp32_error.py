@@ -65,3 +65,20 @@ def test_weights_come_from_the_scores_of_the_forward(be, D):
         return torch.autograd.grad(out, leaves, do)[2]
 
     assert torch.equal(dv(q), dv(torch.zeros_like(q)))
+
+
+@pytest.mark.parametrize("be,D", SHAPES)
+def test_lse_of_one_key_is_its_score(be, D):
+    """Scores of whole numbers are exact: the log-sum-exp of a row of one key is
+    its score times scale log2 e, rounded once."""
+    from vsa_mi355x import mi355x as M
+    nb, H, scale = 5, 3, 0.01
+    g = torch.Generator(device=DEV).manual_seed(be + D)
+    q, k = (torch.randint(-3, 4, (1, H, be * nb, D), generator=g, device=DEV).float()
+            for _ in range(2))
+    sel, vbs = _own_block(H, nb)
+    lse = M.sparse_forward(q, k, k, sel, vbs, be, scale)[1].view(H, nb, be)
+    keys = k.view(H, nb, be, 1, D)[:, :, :1, 0]
+    s = (q.view(H, nb, be, D) * keys).sum(-1)
+    c2 = torch.tensor(scale, dtype=torch.float32) * torch.tensor(math.log2(math.e))
+    assert torch.equal(lse, s * c2.to(DEV))
