@@ -4,23 +4,28 @@
 // padding masks follow the bf16 / fp16 kernels of fine_fwd.hip and
 // fine_bwd.hip with T = fp32.
 //
-// Head dims 64 / 128 run their products on the bf16
-// matrix core: every fp32 operand is the exact sum of three bf16 values, each
-// the upper half of what the ones before leave (mid < 2^-7 hi, lo < 2^-15 hi),
-// and a product is its six largest partial products, accumulated in fp32
-// (mid.lo and lo.mid, on average 2^-25 of the product, are left out: half an
-// fp32 rounding).  A 32x32 tile over 16 dims takes 6 x 32 cycles against
-// 8 x 64 on v_mfma_f32_32x32x2_f32, and its sum is rounded 6 times instead of
-// 16.  Bound by the matrix core: at 12 heads, 16 384 tokens, head dim 128,
-// block 256, topk 8 the forward takes 1.31 ms against 2.89 on the fp32 units,
-// dQ 1.65 against 2.85, dK/dV 2.47 against 4.31 (950 - 1 130 TFLOP/s of bf16
-// products; a large bf16 matrix product reaches 1 126 on this card), and the
-// error against fp64 is 1.0e-6 against 1.1e-6.
+// Head dims 64 / 128 run their products on the bf16 matrix core (the splitting of
+// Henry, Tang and Heinecke, 2019, with three parts): every fp32 operand is the
+// exact sum of three bf16 values, hi and mid rounded to the nearest, and a product
+// is its six largest partial products, accumulated in fp32.  What is left out
+// (mid.lo, lo.mid, lo.lo) has either sign and is at most 2^-24 of a product, half
+// an fp32 rounding.  With parts that were truncated it had the product's sign and
+// reached 2^-21 (dP of near-constant rows off by 4e-7 in common, now 7e-8 rms, 8e-7
+// on the fp32 matrix core), for 1 % less time.  A 32x32 tile over 16 dims takes
+// 6 x 32 cycles against 8 x 64 on v_mfma_f32_32x32x2_f32, and its sum is rounded 6
+// times instead of 16.  Bound by the matrix core and the splitting beside it: at 12
+// heads, 16 384 tokens, head dim 128, block 256, topk 8 the forward takes 1.39 ms
+// against 2.89 on the fp32 units, dQ 1.73 against 2.85, dK/dV 2.56 against 4.31,
+// and the error against fp64 is 1.0e-6 against 1.1e-6.
+//
+// The parts hold an operand's 24 bits from 2^-110 (7.7e-34) up.  Below, up to
+// 2^-133 of each operand is lost (3e-6 rms at 1e-35), bf16's last place; that
+// counts for the backward's dS = P (dP - delta) too, so from |dO| of about 1e-32
+// down, depending on P.
 //
 // The forward and dQ at head_dim 256 (split fragments would exceed a wave's
-// registers) run on
-// v_mfma_f32_32x32x2_f32 (the fp32 matrix core: 1/16 of the bf16 rate, twice
-// the unpacked fp32 VALU rate).  Its operands are one float per lane:
+// registers) run on v_mfma_f32_32x32x2_f32 (the fp32 matrix core: 1/16 of the
+// bf16 rate, twice the unpacked fp32 VALU rate).  Its operands are one float per lane:
 //   A (32 x 2): lane (r, h) = row r, k = h;  B (2 x 32): lane (c, h) = column c, k = h;
 //   C (32 x 32): element i of lane (c, h) = row 8(i/4) + 4h + i%4, column c.
 // A dot product over D dims is D/2 MFMAs; k-step t pairs dim t (h = 0) with
@@ -132,27 +137,37 @@ struct Split8 {
 __device__ __forceinline__ uint32_t pack_hi16(float a, float b) {
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-__device__ __forceinline__ float trunc16(float x) {
-  return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+// Two floats rounded to bf16 (v_cvt_pk_bf16_f32), packed, and the packed two as
+// floats.
+__device__ __forceinline__ uint32_t round_pair(float a, float b) {
+  typedef bf16_t pair __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, pair{(bf16_t)a, (bf16_t)b});
 }
+__device__ __forceinline__ float low_part(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float high_part(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
-// x = hi + mid + lo of a finite x, each the truncation of what is left: the
-// differences are exact and the last one has 8 significant bits.
+// Magnitudes from here on round to a bf16 infinity.
+constexpr float kSplitMax = 0x1.ffp127f;
+
+// x = hi + mid + lo of |x| < kSplitMax: hi and mid are rounded to the nearest,
+// so that what is left is signed and at most half of the last place (|mid| <=
+// 2^-8 |x|, |lo| <= 2^-17 |x|, with x's leading bit); lo has 8 significant bits
+// and is exact.
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   u32x4 hi, mid, lo;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float a = x[2 * e], b = x[2 * e + 1];
-    const float a1 = a - trunc16(a), b1 = b - trunc16(b);
-    const float a2 = a1 - trunc16(a1), b2 = b1 - trunc16(b1);
-    hi[e] = pack_hi16(a, b);
-    mid[e] = pack_hi16(a1, b1);
+    hi[e] = round_pair(a, b);
+    const float a1 = a - low_part(hi[e]), b1 = b - high_part(hi[e]);
+    mid[e] = round_pair(a1, b1);
+    const float a2 = a1 - low_part(mid[e]), b2 = b1 - high_part(mid[e]);
     lo[e] = pack_hi16(a2, b2);
   }
   return {as_vec8<bf16_t>(hi), as_vec8<bf16_t>(mid), as_vec8<bf16_t>(lo)};
 }
 
-// Largest magnitude of the eight (a NaN stays a NaN): split8 needs it finite.
+// Largest magnitude of the eight (a NaN stays a NaN): split8 needs it below kSplitMax.
 __device__ __forceinline__ float absmax8(const float (&x)[8]) {
   float mx = fabsf(x[0]);
 #pragma unroll
@@ -160,18 +175,23 @@ __device__ __forceinline__ float absmax8(const float (&x)[8]) {
   return mx;
 }
 
-// split8 of any values: an infinity or NaN goes into the lo part alone.  lo
-// only meets the other operand's hi part, so inf * y is an infinity of the
-// right sign (NaN for y = 0) as in fp32, where an infinite hi would also meet
-// the zeros and signs of the other operand's mid and lo parts.
+// split8 of any values.  The largest finite ones keep bf16's largest as their hi
+// part.  An infinity or NaN goes into the lo part, which only meets the other
+// operand's hi part, beside a hi part of +-1: inf * y is then an infinity of the
+// right sign (NaN for y = 0), also where y is infinite; an infinite hi part
+// would meet the zeros and signs of the other operand's mid and lo parts.
 __device__ __forceinline__ Split8 split8_any(const float (&x)[8]) {
-  float y[8];
+  constexpr float kMax = 0x1.fep127f;
+  Split8 s;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) y[e] = fabsf(x[e]) < INFINITY ? x[e] : 0.f;
-  Split8 s = split8(y);
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (!(fabsf(x[e]) < INFINITY)) s.lo[e] = (bf16_t)x[e];
+  for (int e = 0; e < 8; ++e) {
+    const bool finite = fabsf(x[e]) < INFINITY;
+    const float y = finite ? x[e] : copysignf(1.0f, x[e]);
+    s.hi[e] = (bf16_t)__builtin_amdgcn_fmed3f(y, -kMax, kMax);
+    const float a1 = y - (float)s.hi[e];
+    s.mid[e] = (bf16_t)a1;
+    s.lo[e] = (bf16_t)(finite ? a1 - (float)s.mid[e] : x[e]);
+  }
   return s;
 }
 
@@ -202,15 +222,18 @@ __device__ __forceinline__ f32x16 mma6_as_ba(const Split8& a, const Split8& b, f
 template <int D>
 __device__ __forceinline__ void load_split(Split8 (&f)[D / 16], const float* __restrict__ row,
                                            int h) {
+  f32x4 raw[D / 16][2];
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      raw[ks][e] = *reinterpret_cast<const f32x4*>(row + 16 * ks + 8 * h + 4 * e);
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks) {
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 8; e += 4) {
-      const f32x4 t = *reinterpret_cast<const f32x4*>(row + 16 * ks + 8 * h + e);
-      x[e] = t[0]; x[e + 1] = t[1]; x[e + 2] = t[2]; x[e + 3] = t[3];
-    }
-    f[ks] = split8_any(x);
+    __builtin_amdgcn_sched_barrier(0);  // one piece's temporaries at a time
+    const float x[8] = {raw[ks][0][0], raw[ks][0][1], raw[ks][0][2], raw[ks][0][3],
+                        raw[ks][1][0], raw[ks][1][1], raw[ks][1][2], raw[ks][1][3]};
+    f[ks] = __any(!(absmax8(x) < kSplitMax)) ? split8_any(x) : split8(x);
   }
 }
 
@@ -226,7 +249,7 @@ struct SplitTile {
 // splits piece i (8 floats of one row) and writes it to the three planes.  The
 // pieces are put between the MFMAs of the product before the tile's own, with
 // no branch among them; finish() writes the tile again, value by value, in the
-// rare case that it holds an infinity or NaN.
+// rare case that it holds an infinity, a NaN or a value that rounds to one.
 template <int D, int NT>
 struct SplitCopy {
   static constexpr int N = kChunk * D / 8 / NT;
@@ -259,7 +282,7 @@ struct SplitCopy {
     store(i, split8(v), tile);
   }
   __device__ __forceinline__ void finish(bf16_t* tile) const {
-    if (!__any(!(mx < INFINITY))) return;
+    if (!__any(!(mx < kSplitMax))) return;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const float v[8] = {buf[i][0][0], buf[i][0][1], buf[i][0][2], buf[i][0][3],
@@ -315,7 +338,7 @@ __device__ __forceinline__ void split_acc_any(const f32x16& acc, Split8 (&s)[2])
 #pragma unroll
   for (int e = 0; e < 16; ++e) x[e >> 3][e & 7] = acc[e];
   const float mx = vmax(absmax8(x[0]), absmax8(x[1]));
-  if (__any(!(mx < INFINITY))) {
+  if (__any(!(mx < kSplitMax))) {
     s[0] = split8_any(x[0]);
     s[1] = split8_any(x[1]);
   } else {
@@ -347,8 +370,6 @@ template <int D, int BE>
 struct SplitCfg {
   static constexpr int ROWS = BE >= 128 ? 128 : 64;
   static constexpr int NT = 2 * ROWS;
-  // waves per SIMD the registers are sized for: the fragments of a row take
-  // 3 D/4 registers (one operand in the forward, two backward)
   // backward: the tiles' loads are issued one product ahead of the product they
   // are put under; a two-wave workgroup (twice the registers of loads a thread)
   // issues them as that product starts
@@ -359,6 +380,8 @@ struct SplitCfg {
   // two-wave workgroup, of which two share a CU, keeps one Q buffer
   static constexpr bool VLO = D == 128;
   static constexpr int QBUF = VLO && NT == 128 ? 1 : 2;
+  // waves per SIMD the registers are sized for: the fragments of a row take
+  // 3 D/4 registers (one operand in the forward, two backward)
   static constexpr int WPE_FWD = D == 64 ? 2 : 1;
   static constexpr int WPE_DQ = D == 64 && BE >= 128 ? 2 : 1;
 };

@@ -19,14 +19,17 @@ The building blocks (pooling, coarse attention + Top-K, CSR inversion, fine
 forward / backward) are exposed as functions so tests can check each kernel.
 
 The kernels exist for block volumes 64 / 128 / 256 and head dims 64 / 128 /
-256; bf16 / fp16 run on the MFMA kernels, fp32 on kernels of its own (no
-rounding below fp32 anywhere on its path).  Other shapes the reference accepts
-on the GPU (volume in [1, 128], head_dim <= 256; triton_impl.py:379-384) run on
-the same kernels after zero-padding each block to the next kernel volume and
-the head dim to the next kernel width; the softmax scale stays 1/sqrt(head_dim)
-of the caller's tensors.  Padded query rows are dropped (and 32 of them together
-are not multiplied), padded keys are masked by the block sizes, padded channels
-are zero in every dot product.
+256; bf16 / fp16 run on the MFMA kernels, fp32 on kernels of its own: inputs,
+sums and results in fp32; products in fp32 at head dim 256, and at 64 / 128 as
+six of the nine partial products of operands split exactly into three bf16
+parts, at most 2^-24 of a product left out (operands below 2^-110 = 7.7e-34
+lose up to 2^-133 each besides).  Other shapes the reference accepts on the GPU
+(volume in [1, 128], head_dim <= 256; triton_impl.py:379-384) run on the same
+kernels after zero-padding each block to the next kernel volume and the head dim
+to the next kernel width; the softmax scale stays 1/sqrt(head_dim) of the
+caller's tensors.  Padded query rows are dropped (and 32 of them together are
+not multiplied), padded keys are masked by the block sizes, padded channels are
+zero in every dot product.
 
 Both ops run a whole pass as one call into the library (``launch``); the
 functions here check, convert and pick the op's sizes.
