@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "fine_f32.h"
+#include "fwd_pieces.h"
 #include "vsa_device.h"
 #include "vsa_launch.h"
 
@@ -43,9 +44,6 @@ struct FwdCfg {
   // waves per SIMD the registers are sized for: head_dim 256 (Q fragments and
   // O accumulators alone take 192 registers) runs one wave per SIMD
   static constexpr int WPE = D == 256 ? 1 : 2;
-  // workgroups a CU holds at block 64: by registers and LDS four (2 waves each)
-  // at head dim 128, eight at 64
-  static constexpr int WG_PER_CU = D == 64 ? 8 : 4;
   static constexpr int TILE = KC * D;              // elements of one K (or V) chunk
   static constexpr int STAGE = 2 * TILE;           // K and V
 };
@@ -824,32 +822,9 @@ static int launch_fwd(const void* q, const void* k, const void* v, const int32_t
   const int grid = (int)(((tiles + 7) / 8) * 8);
   const float c2 = fabsf(scale) * kLog2e;
   const uint32_t qsign = scale < 0.f ? 0x80008000u : 0u;
-  // Workgroups of one head that start together walk their routes (ascending key
-  // blocks) roughly in step and find most K / V tiles in their XCD's L2; left to
-  // start as others end, they drift apart, and a head's K / V does not fit.  At
-  // block 64, which reads the most K / V per product, a long pass (ten times the
-  // workgroups the chip holds at once: the drift adds up) whose heads have
-  // several times the L2 of K / V and whose routes are long is therefore launched
-  // in pieces of the workgroups the chip holds (the last one takes the
-  // remainder).  Whole / in pieces on the op's own routes, head dim 128, top-k an
-  // eighth: 40 heads x 640 blocks 6.90 / 5.50 ms, 24 x 640 3.84 / 3.33, 16 x 640
-  // 2.45 / 2.27, 12 x 1280 8.60 / 6.64, 40 x 400 2.44 / 2.34; head dim 64, 24 x
-  // 1280 8.57 / 7.22.  On skewed routes, which share key blocks as they are, the
-  // lines keep it even (40 x 384 1.84 / 1.83 ms, 24 x 1280 with 48 of them 3.86 /
-  // 3.89, head dim 64 6.51 / 6.52); below them the pieces' ends cost what they
-  // bring: 12 x 624 1.49 / 1.53 ms, 24 x 320 822 / 829 us, skewed routes of 40 in
-  // 1280 3.44 / 3.52 ms, at head dim 64 of 100 in 800 2.47 / 2.60; so they do for
-  // padded rows (20 x 640 blocks of 27, with backward 5.55 / 5.62), at block 128
-  // (16 x 640 7.38 / 7.44) and at head dim 256 (8 x 640 2.66 / 2.70).
-  constexpr int64_t kL2Bytes = 4 << 20;
-  constexpr int64_t kKvBytes = (D == 64 ? 5 : 3) * kL2Bytes;
-  constexpr int kLongRoute = D == 64 ? 160 : 48;
-  const int held = (cu_count() * C::WG_PER_CU + 7) / 8 * 8;
-  const bool pieces = BE == 64 && D <= 128 && rows > BE - 32 && topk >= kLongRoute &&
-                      2 * skv * D * (int64_t)sizeof(T) >= kKvBytes && grid / 10 >= held;
-  const int piece = pieces ? held : grid;
+  const int piece = fwd_piece(D, BE, rows, grid, skv, topk, sizeof(T), cu_count());
   for (int first = 0, n; first < grid; first += n) {
-    n = grid - first - piece < piece ? grid - first : piece;
+    n = fwd_launch(grid, first, piece);
     hipLaunchKernelGGL(kernel, dim3(n), dim3(C::NT), 0, stream,
                        (const T*)q, (const T*)k, (const T*)v, selected, kv_vbs, (T*)out, (T*)fine, lse,
                        (const T*)outc, (const T*)gate, gate_mode, gate_heads, (int)tiles, tph, (int)sq,

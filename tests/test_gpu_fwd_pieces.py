@@ -43,3 +43,22 @@ def test_pieces_equal_single_launches(d, per_cu, kb, tk, be, pieces, off):
             ref = _attend(q[:, :, i * be:(i + n) * be].contiguous(), k, v,
                           sel[:, :, i:i + n].contiguous(), vbs, be)
             assert torch.equal(got[:, :, i * be:(i + n) * be], ref), i
+
+
+def test_token_major_views_in_pieces():
+    """The raster instance of the kernel: all heads in one call, which is split,
+    against nine heads a call, which are not (10 368 and 3 456 workgroups)."""
+    from vsa_mi355x import mi355x as M
+    H, nb, tk, d = 27, 384, 48, 128
+    g = torch.Generator(device=DEV).manual_seed(7)
+    q, k, v = (torch.randn(1, nb * 64, H, d, generator=g, device=DEV).bfloat16() for _ in range(3))
+    vbs = torch.randint(1, 65, (nb,), generator=g, device=DEV, dtype=torch.int32)
+
+    def op(h):
+        views = (x[:, :, h].contiguous().transpose(1, 2) for x in (q, k, v))
+        return M.mi355x_vsa(*views, vbs, vbs, tk, (4, 4, 4))
+
+    with torch.no_grad():
+        got = op(slice(None))
+        for i in range(0, H, 9):
+            assert torch.equal(got[:, i:i + 9], op(slice(i, i + 9))), i
