@@ -88,9 +88,9 @@ __device__ __forceinline__ int acc_row(int i, int h) { return 8 * (i >> 2) + 4 *
 
 // LDS of a pass: the waves' operand tiles, then (the same memory) the partial
 // sums of reduce_rows.
-template <typename T, int DH, int TILES>
+template <typename T, int DH>
 union Shared {
-  T tile[kWaves][TILES][32 * DH];
+  T tile[kWaves][32 * DH];
   float part[kParts][32 * (DH + 1)];
 };
 
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(kNT) void coarse_fwd_mfma_kernel(
     float scale) {
   using E = Elem<T>;
   typedef typename E::vec8 V8;
-  __shared__ __attribute__((aligned(16))) Shared<T, D, 1> sh;
+  __shared__ __attribute__((aligned(16))) Shared<T, D> sh;
   __shared__ float smax[kWaves][32], ssum[kWaves][32];
   const int64_t b = blockIdx.y;
   const int q0 = blockIdx.x * kRows;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(kNT) void coarse_fwd_mfma_kernel(
   f32x16 oacc[D / 32];
 #pragma unroll
   for (int mt = 0; mt < D / 32; ++mt) oacc[mt] = f32x16{};
-  T* vt = sh.tile[wave][0];
+  T* vt = sh.tile[wave];
   auto add_pv = [&](const float (&p)[16]) {  // out_c^T += V^T P^T, V in vt
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(kNT) void coarse_bwd_rows_mfma_kernel(
   using E = Elem<T>;
   typedef typename E::vec8 V8;
   constexpr int DH = D < 128 ? D : 128;
-  __shared__ __attribute__((aligned(16))) Shared<T, DH, 1> sh;
+  __shared__ __attribute__((aligned(16))) Shared<T, DH> sh;
   __shared__ float ssum[kWaves][32];
   const int64_t b = blockIdx.y;
   const int q0 = blockIdx.x * kRows, d_off = blockIdx.z * DH;
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(kNT) void coarse_bwd_rows_mfma_kernel(
   f32x16 qacc[DH / 32];
 #pragma unroll
   for (int mt = 0; mt < DH / 32; ++mt) qacc[mt] = f32x16{};
-  T* kt_ = sh.tile[wave][0];
+  T* kt_ = sh.tile[wave];
   RowStage<T, D, DH> kst;
   auto finish_tile = [&](int kt, float (&dp)[16], const float (&p)[16], float rsum, bool more) {
 #pragma unroll
@@ -607,7 +607,7 @@ __global__ __launch_bounds__(kNT) void coarse_bwd_cols_mfma_kernel(
   using E = Elem<T>;
   typedef typename E::vec8 V8;
   constexpr int DH = D < 128 ? D : 128;
-  __shared__ __attribute__((aligned(16))) Shared<T, DH, 1> sh;
+  __shared__ __attribute__((aligned(16))) Shared<T, DH> sh;
   const int64_t b = blockIdx.y;
   const bool is_v = blockIdx.z & 1;
   const int k0 = blockIdx.x * kRows, d_off = (blockIdx.z >> 1) * DH;
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(kNT) void coarse_bwd_cols_mfma_kernel(
   f32x16 acc[DH / 32];
 #pragma unroll
   for (int mt = 0; mt < DH / 32; ++mt) acc[mt] = f32x16{};
-  T* tile = sh.tile[wave][0];
+  T* tile = sh.tile[wave];
   for (int t = wave; t < ntile; t += kWaves) {
     // B operand: the weights [q][key r] of the 16 queries this lane feeds (rows
     // past the end are clamped, loaded and zeroed: a load under the condition
