@@ -13,10 +13,12 @@
 // reached 2^-21 (dP of near-constant rows off by 4e-7 in common, now 7e-8 rms, 8e-7
 // on the fp32 matrix core), for 1 % less time.  A 32x32 tile over 16 dims takes
 // 6 x 32 cycles against 8 x 64 on v_mfma_f32_32x32x2_f32, and its sum is rounded 6
-// times instead of 16.  Bound by the matrix core and the splitting beside it: at 12
-// heads, 16 384 tokens, head dim 128, block 256, topk 8 the forward takes 1.39 ms
-// against 2.89 on the fp32 units, dQ 1.73 against 2.85, dK/dV 2.56 against 4.31,
-// and the error against fp64 is 1.0e-6 against 1.1e-6.
+// times instead of 16.  At 12 heads, 16 384 tokens, head dim 128, block 256, topk 8
+// the forward takes 1.39 ms against 2.89 on the fp32 units, dQ 1.73 against 2.85,
+// dK/dV 2.56 against 4.31, and the error against fp64 is 1.0e-6 against 1.1e-6.
+// Bound by one wave per SIMD at head dim 128 (registers): the matrix core is busy
+// 40 / 48 / 48 % of the time and the vector unit, which splits operands, 36 / 33 /
+// 26 %, mostly one after the other.
 //
 // The parts hold an operand's 24 bits from 2^-110 (7.7e-34) up.  Below, up to
 // 2^-133 of each operand is lost (3e-6 rms at 1e-35), bf16's last place; that
