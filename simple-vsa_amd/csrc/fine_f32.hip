@@ -334,7 +334,8 @@ __device__ __forceinline__ Split8 split_acc(const f32x16& acc, int kk) {
   return split8(x);
 }
 
-// The same of a tile of any values (dS, where an infinite dO or V makes some).
+// The same of a tile of any values (dS, where an infinite dO or V makes some); the
+// look over the tile takes 1 % of dQ and dK / dV.
 __device__ __forceinline__ void split_acc_any(const f32x16& acc, Split8 (&s)[2]) {
   float x[2][8];
 #pragma unroll
@@ -419,8 +420,11 @@ struct RouteCursor {
 // more than kMaxSlack: O is rescaled on few chunks, and the exponents of the
 // largest weights stay near 0, where fp32 resolves them.  The weights are kept
 // as 2^-kMaxSlack of their value, at most 1, so that no product passes v's
-// largest.  The next V tile is split and written under the S products, the next
-// K tile under the O products: one buffer each and two barriers a chunk.
+// largest.  (An offset 8 above the max took 3 % less, 1.355 against 1.397 ms at 12
+// heads, 16 384 tokens, head dim 128, and left each weight with a rounding of up to
+// 3e-7; a slack of 2 rescales often enough to cost 2 % more, 6 is as fast as 4.)
+// The next V tile is split and written under the S products, the next K tile under
+// the O products: one buffer each and two barriers a chunk.
 // ---------------------------------------------------------------------------
 constexpr int kMaxSlack = 4;
 
